@@ -32,7 +32,7 @@
 //   JQ, G, Qtp [K][5][np]        point n + ncg*(m + ncg*l)
 //   T, FV      [K][6][5][nf]     face traces, face f-1, point i + ncg*j
 //   QA, FI, FT [M][5][nf]        per mortar (master face indexing)
-//   metrics    jacob [K][npm], gmetg [K][9][npm], gmet_d [K][3][nsm],
+//   metrics    jacob [K][npm], gmetg [K][9][npm], gmet [K][3 grids][3][nsm],
 //              nhat [M][3][nfm], norm [M][nfm]; npm = np (per point) or 1
 //              (per element, affine meshes) -- selected by the stride ms.
 #include <hip/hip_runtime.h>
@@ -53,14 +53,9 @@ namespace {
 
 constexpr int NEQ = 5;
 constexpr int BLOCK = 256;
-// Fused volume kernel: one element per workgroup.  FP64 at p = 7, 8 holds
-// 105-151 KB of LDS per element, so one workgroup fills a CU, and its
-// matrix-core tiles (48, 63 per direction) need 1024 work-items (16 lanes
-// each); at p <= 6 every direction has at most 26 tiles, so 512 work-items
-// hold them all and two elements (<= 72 KB each) share a CU.  The FP32
-// modes (75 KB at p = 8) fit two workgroups of 512 per CU.
-template <int P, int PM>
-constexpr int vblock() { return (PM == 0 && P >= 7) ? 1024 : 512; }
+// Mixed-precision volume kernel: one element per workgroup; the FP32 tiles
+// (75 KB at p = 8) let two workgroups of 512 share a CU.
+constexpr int VBLOCK = 512;
 
 // operators for every order p = 1..8, indexed [p]
 __constant__ double c_D[9][90];   // D[k*nc + j]
@@ -84,8 +79,8 @@ __constant__ double c_dct3[9][81];
 // name itself.
 __device__ __align__(256) double scratch[DSEM_NOALLOC_SCRATCH_BYTES / sizeof(double)];
 
-// Contraction arithmetic of the volume kernel, by precision mode:
-//   PM 0  FP64 (the drop-in path);
+// Contraction arithmetic of the mixed-precision volume kernel, by mode (FP64,
+// the drop-in path, has its own kernel: volume.inc):
 //   PM 1  FP32 multiply-add, FP32 accumulation;
 //   PM 2  BF16 split products: a*b ~ ah*bh + ah*bl + al*bh with
 //         x = xh + xl, xh = bf16(x), xl = bf16(x - xh); each product of two
@@ -98,12 +93,6 @@ struct Ctr {
     using T = float;
     using A = float;
 };
-template <>
-struct Ctr<0> {
-    using T = double;
-    using A = double;
-};
-
 __device__ __forceinline__ float bf16_round(float x)
 {
     unsigned u = __float_as_uint(x);
@@ -115,9 +104,7 @@ template <int PM>
 __device__ __forceinline__ typename Ctr<PM>::A mac(typename Ctr<PM>::T a, typename Ctr<PM>::T b,
                                                     typename Ctr<PM>::A acc)
 {
-    if constexpr (PM == 0) {
-        return fma(a, b, acc);
-    } else if constexpr (PM == 1) {
+    if constexpr (PM == 1) {
         return fmaf(a, b, acc);
     } else {
         const float ah = bf16_round(a), al = bf16_round(a - ah);
@@ -126,22 +113,6 @@ __device__ __forceinline__ typename Ctr<PM>::A mac(typename Ctr<PM>::T a, typena
         acc = fmaf(ah, bl, acc);
         return fmaf(al, bh, acc);
     }
-}
-
-template <int PM>
-__device__ __forceinline__ typename Ctr<PM>::T opB(int p, int idx)
-{
-    if constexpr (PM == 0) return c_B[p][idx]; else return c_Bf[p][idx];
-}
-template <int PM>
-__device__ __forceinline__ typename Ctr<PM>::T opD(int p, int idx)
-{
-    if constexpr (PM == 0) return c_D[p][idx]; else return c_Df[p][idx];
-}
-template <int PM>
-__device__ __forceinline__ typename Ctr<PM>::T opM(int p, int idx)
-{
-    if constexpr (PM == 0) return c_M[p][idx]; else return c_Mf[p][idx];
 }
 
 template <int P>
@@ -154,7 +125,7 @@ struct Sz {
 struct DevMesh {
     int K, M, ms;                 // ms: 1 per-point metrics, 0 per-element
     int rot;                      // some mortar face is rotated (orientation != 0)
-    const double *jacob, *gmetg, *gmet0, *gmet1, *gmet2;
+    const double *jacob, *gmetg, *gmet;
     const int *e2m;               // [K][6] (mortar << 4) | (map << 1) | side, see e2m_mortar
     const int *m_elem, *m_face, *m_sign, *m_nsign;
     const int *m_orient;          // [M] slave orientation 0..7, or null when every mortar is aligned
@@ -397,7 +368,7 @@ __global__ __launch_bounds__(BLOCK) void k_face_inv(const double *__restrict__ T
     }
 }
 
-// Line contractions of the FP64 volume kernel on the matrix cores.
+// Line contractions of the adjoint volume kernel on the matrix cores.
 // v_mfma_f64_4x4x4f64 runs four independent 4x4x4 products per wave.  Lane l
 // (c = l%4, blk = (l/4)%4, r = l/16) supplies A_blk[c][r] and B_blk[r][c]
 // and receives D_blk[r][c] (layout measured on gfx950).  With A = four rows
@@ -477,75 +448,24 @@ __device__ __forceinline__ double mf_line(const double *fld, const MfLane<P, ROW
     return t;
 }
 
-// One staggered grid D of the fused volume kernel: fluxes at the nc*ncg^2
-// points of grid D into LDS (interior) or the viscous face traces (faces),
-// then the interior part of the divergence along D added into acc.
-// MF (FP64 only): the interpolation of Q and the prolongation of the 15
-// gradients run on the matrix cores (mf_line), one point per lane; otherwise
-// each work-item forms its point's 9-term sums on the vector ALUs.
-// Flux of the lane's staggered point in the matrix-core form, held in
-// registers until every wave is past the previous divergence pass.
-struct LaneFlux {
-    double f[5];
-    int s;
-    bool store;
-};
-
-template <int P, int D, int PM, bool MF>
-__device__ __forceinline__ LaneFlux volume_grid(const DevMesh &m, const DevPhys &ph, const double *__restrict__ QA,
+// One staggered grid D of the mixed-precision volume kernel: fluxes at the
+// nc*ncg^2 points of grid D into LDS (interior) or the viscous face traces
+// (faces).
+template <int P, int D, int PM>
+__device__ __forceinline__ void volume_grid(const DevMesh &m, const DevPhys &ph, const double *__restrict__ QA,
                                             const double *__restrict__ muh, const double *__restrict__ nut,
                                             double *__restrict__ FV, double *__restrict__ Slag,
                                             const typename Ctr<PM>::T *sQ,
                                             const typename Ctr<PM>::T *sG, typename Ctr<PM>::T *sF,
-                                            const double *sBar, const typename Ctr<PM>::T *sD,
-                                            const typename Ctr<PM>::T *sB, const double *sDint, int e,
-                                            const int *e2m_e, const MfLane<P> &ml, int tid)
+                                            const double *sBar, const typename Ctr<PM>::T *sB, int e,
+                                            const int *e2m_e, int tid)
 {
     using S = Sz<P>;
     using CT = typename Ctr<PM>::T;
     using CA = typename Ctr<PM>::A;
-    static_assert(!MF || PM == 0, "matrix-core contractions are FP64 only");
-    constexpr int VBLOCK = vblock<P, PM>();
-    static_assert(!MF || MfTiles<P>::NT <= VBLOCK / 16, "one tile per 16 lanes in one pass");
-    constexpr int KS = MfTiles<P>::KS;
     const int nsm = m.ms ? S::NS : 1, nfm = m.ms ? S::NF : 1;
-    const double *gmd = (D == 0 ? m.gmet0 : (D == 1 ? m.gmet1 : m.gmet2)) + (size_t)e * 3 * nsm;
-    // Matrix-core form: the lane's point is fixed, so its metric row and face
-    // values are loaded before the barrier and arrive while the other waves
-    // finish the previous pass.
-    int mf_s = 0;
-    double mf_g[3] = {0.0, 0.0, 0.0}, mf_qa[5] = {0.0, 0.0, 0.0, 0.0, 0.0};
-    double mf_nrm = 1.0, mf_nut = 0.0, mf_muh = 0.0;
-    if constexpr (MF) {
-        const int a = ml.line % S::NCG, b = ml.line / S::NCG;
-        mf_s = sidx<P>(D, ml.valid ? ml.j : 0, a, b);
-        if (ml.valid) {
-#pragma unroll
-            for (int i = 0; i < 3; ++i) mf_g[i] = gmd[i * nsm + mf_s * m.ms];
-            if (nut) mf_nut = nut[((size_t)e * 3 + D) * S::NS + mf_s];
-            if (muh) mf_muh = muh[((size_t)e * 3 + D) * S::NS + mf_s];
-            if (ml.j == 0 || ml.j == S::NC - 1) {
-                const int c = e2m_e[face_of<P>(D, ml.j) - 1];
-                const int mo = e2m_mortar(c);
-                const int q = m.rot ? orient_point<S::NCG>(e2m_map(c), a + S::NCG * b) : a + S::NCG * b;
-#pragma unroll
-                for (int v = 0; v < 5; ++v) mf_qa[v] = QA[((size_t)mo * NEQ + v) * S::NF + q];
-                mf_nrm = m.norm[(size_t)mo * nfm + q * m.ms];
-            }
-        }
-    }
-    // Matrix-core form, grids 1 and 2: a lane's flux waits in registers, and the
-    // barrier that keeps the previous divergence pass's reads of sF ahead of
-    // this grid's writes comes after the arithmetic, so the two passes overlap
-    // across waves.  Grid 0 (and the vector form) waits here: sG complete /
-    // previous divergence pass done with sF.
-    double mf_f[5] = {0.0, 0.0, 0.0, 0.0, 0.0};
-    int mf_fs = 0;
-    bool mf_fstore = false;
-    if constexpr (!MF || D == 0) __syncthreads();
-    // Matrix-core form: one pass, every lane of an active wave takes part in
-    // the contractions (the tiles need all 64 lanes); only lanes that own a
-    // point store.  Vector form: work-items stride over the points.
+    const double *gmd = m.gmet + ((size_t)e * 3 + D) * 3 * nsm;
+    __syncthreads();   // sG complete / previous divergence pass done with sF
     // FP32 mode (PM 1): the 20 contractions of a point (5 interpolated state
     // fields, 15 prolonged gradients) run on v_mfma_f32_4x4x1f32.  Each 4x4
     // block is one line and four consecutive Lobatto rows j; lane i of a
@@ -554,37 +474,26 @@ __device__ __forceinline__ LaneFlux volume_grid(const DevMesh &m, const DevPhys 
     // 4 ch .. 4 ch + 3 at its own point (D column i, rows in the four
     // result registers).  Five chains of ncg steps give all 20 fields at the
     // lane's point; passes cover the ncg^2 lines x ceil(nc/4) row groups.
+    // BF16x3 (PM 2): vector code, work-items stride over the points.
     constexpr bool MF32 = (PM == 1);
     constexpr int JG = (S::NC + 3) / 4;                       // row groups per line
     constexpr int NB32 = S::NCG * S::NCG * JG;                // blocks per grid
     constexpr int NPASS32 = (NB32 + VBLOCK / 4 - 1) / (VBLOCK / 4);
-    const int w0 = (MF || MF32) ? 0 : tid;
-    const int wend = MF ? (ml.wave_active ? 1 : 0) : (MF32 ? NPASS32 : S::NS);
-    const int wstep = (MF || MF32) ? 1 : VBLOCK;
+    const int w0 = MF32 ? 0 : tid;
+    const int wend = MF32 ? NPASS32 : S::NS;
+    const int wstep = MF32 ? 1 : VBLOCK;
 #pragma unroll 1
     for (int w = w0; w < wend; w += wstep) {
         int a, b, j;
         bool valid = true;
-        int off[KS];
-        int line32 = 0;
         if constexpr (MF32) {
             const int blk = w * (VBLOCK / 4) + tid / 4;
             const int line = blk / JG;
             j = 4 * (blk % JG) + tid % 4;
             valid = line < S::NF && j < S::NC;
-            line32 = line < S::NF ? line : 0;                 // past the last line: read line 0, keep nothing
+            const int line32 = line < S::NF ? line : 0;       // past the last line: read line 0, keep nothing
             a = line32 % S::NCG;
             b = line32 / S::NCG;
-        } else if constexpr (MF) {
-            j = ml.j;
-            a = ml.line % S::NCG;
-            b = ml.line / S::NCG;
-            valid = ml.valid;
-#pragma unroll
-            for (int ks = 0; ks < KS; ++ks) {
-                const int k = 4 * ks + ml.r;
-                off[ks] = gidx<P>(D, k < S::NCG ? k : S::NCG - 1, a, b);   // in range (ml.line is 0 past the last line)
-            }
         } else {
             const int s0 = w;
             if (D == 0) { j = s0 % S::NC; a = (s0 / S::NC) % S::NCG; b = s0 / (S::NC * S::NCG); }
@@ -593,25 +502,23 @@ __device__ __forceinline__ LaneFlux volume_grid(const DevMesh &m, const DevPhys 
         }
         const int q = a + S::NCG * b;
         const int jc = valid ? j : 0;
-        const int s = MF ? mf_s : sidx<P>(D, jc, a, b);
+        const int s = sidx<P>(D, jc, a, b);
         const bool face = (jc == 0 || jc == S::NC - 1);
         const int fc = face_of<P>(D, jc);
         const int mo = e2m_mortar(e2m_e[fc - 1]);
         const int qm = m.rot ? orient_point<S::NCG>(e2m_map(e2m_e[fc - 1]), q) : q;   // the face point on the mortar
-        // Vector form: the point's metric row, and its line's face average and
-        // norm (every lane: face_of names a face for any j, and interior lanes
-        // hit the face lane's cache lines), requested before the contractions
-        // instead of one wait each at their use
+        // The point's metric row, and its line's face average and norm (every
+        // lane: face_of names a face for any j, and interior lanes hit the
+        // face lane's cache lines), requested before the contractions instead
+        // of one wait each at their use
         double vg[3] = {0.0, 0.0, 0.0}, vqa[5] = {0.0, 0.0, 0.0, 0.0, 0.0}, vnrm = 1.0;
-        if constexpr (!MF) {
 #pragma unroll
-            for (int i = 0; i < 3; ++i) vg[i] = gmd[i * nsm + s * m.ms];
+        for (int i = 0; i < 3; ++i) vg[i] = gmd[i * nsm + s * m.ms];
 #pragma unroll
-            for (int v = 0; v < 5; ++v) vqa[v] = QA[((size_t)mo * NEQ + v) * S::NF + qm];
-            vnrm = m.norm[(size_t)mo * nfm + qm * m.ms];
-        }
+        for (int v = 0; v < 5; ++v) vqa[v] = QA[((size_t)mo * NEQ + v) * S::NF + qm];
+        vnrm = m.norm[(size_t)mo * nfm + qm * m.ms];
         double Qv[5];
-        CT Bj[MF ? 1 : S::NCG];
+        CT Bj[S::NCG];
         float fld32[MF32 ? 20 : 1];
         if constexpr (MF32) {
             typedef float f4 __attribute__((ext_vector_type(4)));
@@ -634,12 +541,6 @@ __device__ __forceinline__ LaneFlux volume_grid(const DevMesh &m, const DevPhys 
             }
 #pragma unroll
             for (int v = 0; v < 5; ++v) Qv[v] = face ? vqa[v] : sBar[v] + (double)fld32[v];
-        } else if constexpr (MF) {
-#pragma unroll
-            for (int v = 0; v < 5; ++v) {
-                const double t = mf_line<P>(sQ + v * S::NP, ml, off);
-                Qv[v] = face ? mf_qa[v] : t;
-            }
         } else {
 #pragma unroll
             for (int k = 0; k < S::NCG; ++k) Bj[k] = sB[j * S::NCG + k];
@@ -651,7 +552,7 @@ __device__ __forceinline__ LaneFlux volume_grid(const DevMesh &m, const DevPhys 
                     CA u = 0;
 #pragma unroll
                     for (int k = 0; k < S::NCG; ++k) u = mac<PM>(Bj[k], sQ[v * S::NP + gidx<P>(D, k, a, b)], u);
-                    if constexpr (PM == 0) Qv[v] = u; else Qv[v] = sBar[v] + (double)u;
+                    Qv[v] = sBar[v] + (double)u;
                 }
                 if (v == 1 || v == 3) __builtin_amdgcn_sched_barrier(0);
             }
@@ -660,28 +561,22 @@ __device__ __forceinline__ LaneFlux volume_grid(const DevMesh &m, const DevPhys 
 #pragma unroll
             for (int v = 0; v < 5; ++v) Slag[(((size_t)e * 3 + D) * NEQ + v) * S::NS + s] = Qv[v];
         }
-        if constexpr (MF) {
-            if (!valid) { Qv[0] = 1.0; Qv[1] = Qv[2] = Qv[3] = 0.0; Qv[4] = 1.0; }   // no point: keep the arithmetic finite
-        }
         const Prim pr = primitives(ph, Qv);
         // Velocity and temperature gradients, one direction c at a time: the
         // prolonged conservative gradient dQ/dx_c (5 fields) is turned into
         // (du/dx_c, dv/dx_c, dw/dx_c, dT/dx_c) and folded into the symmetric
-        // velocity-gradient sums.  Unrolled in the matrix-core form (the next
-        // direction's loads overlap this one's arithmetic, measured 8 % faster);
-        // one direction at a time in the vector form, whose registers would spill.
+        // velocity-gradient sums.  One direction at a time in the vector form,
+        // whose registers would spill.
         double Sxx = 0.0, Syy = 0.0, Szz = 0.0, Sxy = 0.0, Sxz = 0.0, Syz = 0.0, div = 0.0;
         double Tx = 0.0, Ty = 0.0, Tz = 0.0;
-        constexpr int CUNROLL = (MF || MF32) ? 3 : 1;   // MF32: the fields are in registers already
+        constexpr int CUNROLL = MF32 ? 3 : 1;   // MF32: the fields are in registers already
 #pragma unroll CUNROLL
         for (int c = 0; c < 3; ++c) {
             double Gc[5];
 #pragma unroll
             for (int v = 0; v < 5; ++v) {
                 const CT *gl = sG + (c * 5 + v) * S::NP;
-                if constexpr (MF) {
-                    Gc[v] = mf_line<P>(gl, ml, off);
-                } else if constexpr (MF32) {
+                if constexpr (MF32) {
                     (void)gl;
                     Gc[v] = (double)fld32[5 + c * 5 + v];
                 } else {
@@ -707,11 +602,9 @@ __device__ __forceinline__ LaneFlux volume_grid(const DevMesh &m, const DevPhys 
         }
         if (valid) {
             double amu = 1.0;
-            if (nut) amu = amu + (MF ? mf_nut : nut[((size_t)e * 3 + D) * S::NS + s]) * Qv[0];   // static Smagorinsky
-            if (muh) amu = amu + (MF ? mf_muh : muh[((size_t)e * 3 + D) * S::NS + s]);
-            const double g0 = MF ? mf_g[0] : vg[0];
-            const double g1 = MF ? mf_g[1] : vg[1];
-            const double g2 = MF ? mf_g[2] : vg[2];
+            if (nut) amu = amu + nut[((size_t)e * 3 + D) * S::NS + s] * Qv[0];   // static Smagorinsky
+            if (muh) amu = amu + muh[((size_t)e * 3 + D) * S::NS + s];
+            const double g0 = vg[0], g1 = vg[1], g2 = vg[2];
             double rv[5];
             {
                 // Stokes stress and Fourier heat flux (x/y/z_vis_flux, PhysLib.f90:464-470)
@@ -731,47 +624,15 @@ __device__ __forceinline__ LaneFlux volume_grid(const DevMesh &m, const DevPhys 
             if (face) {
                 // r / norm as one reciprocal and five products (a rounding apart
                 // from five divisions, which every wave with a face lane paid)
-                const double rn = 1.0 / (MF ? mf_nrm : vnrm);
+                const double rn = 1.0 / vnrm;
 #pragma unroll
                 for (int v = 0; v < 5; ++v) FV[(((size_t)e * 6 + fc - 1) * NEQ + v) * S::NF + q] = rv[v] * rn;
             } else {
                 double fi[5];
                 euler_from_primitive(pr, Qv, g0, g1, g2, fi);
-                if constexpr (MF) {
 #pragma unroll
-                    for (int v = 0; v < 5; ++v) mf_f[v] = fi[v] - rv[v] * ph.inv_re;
-                    mf_fs = s;
-                    mf_fstore = true;
-                } else {
-#pragma unroll
-                    for (int v = 0; v < 5; ++v) {
-                        if constexpr (PM == 0) sF[v * S::NS + s] = fi[v] - rv[v] * ph.inv_re;
-                        else sF[v * S::NS + s] = (CT)((fi[v] - rv[v] * ph.inv_re) - sBar[5 + D * 5 + v]);
-                    }
-                }
+                for (int v = 0; v < 5; ++v) sF[v * S::NS + s] = (CT)((fi[v] - rv[v] * ph.inv_re) - sBar[5 + D * 5 + v]);
             }
-        }
-    }
-    LaneFlux lf;
-#pragma unroll
-    for (int v = 0; v < 5; ++v) lf.f[v] = mf_f[v];
-    lf.s = mf_fs;
-    lf.store = mf_fstore;
-    return lf;
-}
-
-// Grid D's fluxes into sF.  The matrix-core form stores its lanes' fluxes
-// once every wave is past the previous divergence pass.  On return every
-// wave is past grid D's point pass (its reads of sQ and sG).
-template <int P, int D, int PM, bool MF>
-__device__ __forceinline__ void volume_publish(const LaneFlux &lf, typename Ctr<PM>::T *sF)
-{
-    using S = Sz<P>;
-    if constexpr (MF) {
-        if constexpr (D > 0) __syncthreads();   // every wave is past the previous divergence pass
-        if (lf.store) {
-#pragma unroll
-            for (int v = 0; v < 5; ++v) sF[v * S::NS + lf.s] = lf.f[v];
         }
     }
     __syncthreads();   // fluxes of this grid complete
@@ -782,12 +643,11 @@ __device__ __forceinline__ void volume_publish(const LaneFlux &lf, typename Ctr<
 template <int P, int D, int PM>
 __device__ __forceinline__ void volume_div(const typename Ctr<PM>::T *sF, const typename Ctr<PM>::T *sD,
                                            const double *sBar, const double *sDint, int tid,
-                                           double (&acc)[(Sz<P>::NP + vblock<P, PM>() - 1) / vblock<P, PM>()][5])
+                                           double (&acc)[(Sz<P>::NP + VBLOCK - 1) / VBLOCK][5])
 {
     using S = Sz<P>;
     using CT = typename Ctr<PM>::T;
     using CA = typename Ctr<PM>::A;
-    constexpr int VBLOCK = vblock<P, PM>();
     constexpr int R = (S::NP + VBLOCK - 1) / VBLOCK;
 #pragma unroll
     for (int r = 0; r < R; ++r) {
@@ -805,8 +665,7 @@ __device__ __forceinline__ void volume_div(const typename Ctr<PM>::T *sF, const 
                 CA t = 0;
 #pragma unroll
                 for (int j = 1; j < S::NC - 1; ++j) t = mac<PM>(Dk[j], sF[v * S::NS + sidx<P>(D, j, a, b)], t);
-                if constexpr (PM == 0) acc[r][v] -= t;
-                else acc[r][v] -= (double)t + sBar[5 + D * 5 + v] * sDint[k];
+                acc[r][v] -= (double)t + sBar[5 + D * 5 + v] * sDint[k];
             }
         }
     }
@@ -822,14 +681,26 @@ __device__ __forceinline__ void volume_div(const typename Ctr<PM>::T *sF, const 
 // every lane of the wave.
 typedef __attribute__((address_space(3))) void *LdsPtr;
 
-__device__ __forceinline__ void lds_dword(const void *src, void *lds_wave_base)
+// LDS byte address of an object in shared memory.
+__device__ __forceinline__ unsigned lds_addr(const void *p) { return (unsigned)(size_t)(LdsPtr)p; }
+
+// lds: LDS byte address of the wave's first dword, the same for every lane
+__device__ __forceinline__ void lds_dword(const void *src, unsigned lds)
 {
-    const unsigned l = __builtin_amdgcn_readfirstlane((unsigned)(size_t)(LdsPtr)lds_wave_base);
+    const unsigned l = __builtin_amdgcn_readfirstlane(lds);
     // The LDS base goes in through the {m0} operand constraint: the compiler
     // writes M0 itself and knows the copy reads it, so no value of its own is
     // kept there across the copy.  The s_nop separates that write from the
     // copy's use of M0.
     asm volatile("s_nop 0\n\tglobal_load_lds_dword %0, off" : : "v"(src), "{m0}"(l) : "memory");
+}
+
+// The same with a scalar base address (uniform over the wave) and a byte
+// offset per lane.
+__device__ __forceinline__ void lds_dword_s(const void *src, unsigned off, unsigned lds)
+{
+    const unsigned l = __builtin_amdgcn_readfirstlane(lds);
+    asm volatile("s_nop 0\n\tglobal_load_lds_dword %0, %1" : : "v"(off), "s"(src), "{m0}"(l) : "memory");
 }
 
 // s_waitcnt immediate of gfx9 for vmcnt(0) alone (expcnt 7, lgkmcnt 15).
@@ -841,69 +712,16 @@ __device__ __forceinline__ void lds_copies_done()
     asm volatile("s_waitcnt vmcnt(0)" : : : "memory");
 }
 
-// The next element's volume inputs, copied straight into LDS while the
-// current element finishes: raw J*Q into sQ ([v][pt]), 1/J at every Gauss
-// point into sJ, and the six faces' averages (face f+1 at [f][v][q],
-// gathered by the mortars of the element's e2m entries e2m_e) into sA.
-// Every wave copies 64-dword chunks w, w + NW, ...; each wave waits for its
-// copies (lds_copies_done) before the barrier that publishes them.
-template <int P>
-__device__ __forceinline__ void volume_inputs_lds(const double *__restrict__ JQ, const double *__restrict__ QA,
-                                                  const DevMesh &m, int e, const int *e2m_e, int tid,
-                                                  double *sQ, double *sJ, double *sA)
-{
-    using S = Sz<P>;
-    constexpr int NW = vblock<P, 0>() / 64;
-    constexpr int NQV = NEQ * S::NP, NAV = 6 * NEQ * S::NF;
-    constexpr int DQ = 2 * NQV, DJ = 2 * S::NP, DA = 2 * NAV;   // dwords
-    constexpr int CQ = (DQ + 63) / 64, CJ = (DJ + 63) / 64, CA = (DA + 63) / 64;   // 64-dword chunks
-    const int lane = tid % 64;
-    const int w = __builtin_amdgcn_readfirstlane(tid / 64);
-    // mortars first, before any copy is in flight
-    int mo6[6], map6[6];
-#pragma unroll
-    for (int g = 0; g < 6; ++g) {
-        mo6[g] = e2m_mortar(e2m_e[g]);
-        map6[g] = e2m_map(e2m_e[g]);
-    }
-    const char *q = (const char *)(JQ + (size_t)e * NQV);
-    const char *jac = (const char *)(m.jacob + (size_t)e * (m.ms ? S::NP : 1));
-#pragma unroll
-    for (int u = 0; u < (CQ + NW - 1) / NW; ++u) {
-        const int c = w + u * NW, d = c * 64 + lane;
-        if (d < DQ) lds_dword(q + 4 * d, (char *)sQ + 256 * c);
-    }
-#pragma unroll
-    for (int u = 0; u < (CJ + NW - 1) / NW; ++u) {
-        const int c = w + u * NW, d = c * 64 + lane;
-        if (d < DJ) lds_dword(jac + 8 * ((d >> 1) * m.ms) + 4 * (d & 1), (char *)sJ + 256 * c);
-    }
-#pragma unroll
-    for (int u = 0; u < (CA + NW - 1) / NW; ++u) {
-        const int c = w + u * NW, d = c * 64 + lane;
-        const int i = d >> 1, f = i / (NEQ * S::NF), vq = i % (NEQ * S::NF);
-        int mo = mo6[0], mp = map6[0];
-#pragma unroll
-        for (int g = 1; g < 6; ++g) {
-            mo = f == g ? mo6[g] : mo;
-            mp = f == g ? map6[g] : mp;
-        }
-        const int vqm = m.rot ? (vq / S::NF) * S::NF + orient_point<S::NCG>(mp, vq % S::NF) : vq;
-        if (d < DA) lds_dword((const char *)(QA + (size_t)mo * NEQ * S::NF + vqm) + 4 * (d & 1), (char *)sA + 256 * c);
-    }
-}
-
 // Global loads of one element's state and 1/J and of its six faces'
 // averages, all issued before any use.
-template <int P, int PM>
+template <int P>
 __device__ __forceinline__ void volume_inputs(const double *__restrict__ JQ, const double *__restrict__ QA,
                                               const DevMesh &m, int e, int tid,
-                                              double (&qv)[(NEQ * Sz<P>::NP + vblock<P, PM>() - 1) / vblock<P, PM>()],
-                                              double (&jv)[(NEQ * Sz<P>::NP + vblock<P, PM>() - 1) / vblock<P, PM>()],
-                                              double (&av)[(6 * NEQ * Sz<P>::NF + vblock<P, PM>() - 1) / vblock<P, PM>()])
+                                              double (&qv)[(NEQ * Sz<P>::NP + VBLOCK - 1) / VBLOCK],
+                                              double (&jv)[(NEQ * Sz<P>::NP + VBLOCK - 1) / VBLOCK],
+                                              double (&av)[(6 * NEQ * Sz<P>::NF + VBLOCK - 1) / VBLOCK])
 {
     using S = Sz<P>;
-    constexpr int VBLOCK = vblock<P, PM>();
     constexpr int NQV = NEQ * S::NP, NAV = 6 * NEQ * S::NF;
     constexpr int NQI = (NQV + VBLOCK - 1) / VBLOCK, NAI = (NAV + VBLOCK - 1) / VBLOCK;
     const double *q = JQ + (size_t)e * NEQ * S::NP;
@@ -937,337 +755,175 @@ __device__ __forceinline__ void volume_inputs(const double *__restrict__ JQ, con
     }
 }
 
-// Fused volume kernel: Gauss-point gradients into LDS (Gauss_Deriv,
-// SolnDerivsc.f90:14-83), then for each staggered grid the interpolated
-// state, prolonged gradients, contravariant Euler + viscous fluxes, the
-// viscous face traces r/norm and the interior part of the divergence.
-//
-// Mixed modes (PM 1, 2): the LDS tiles hold FP32 values and the
-// contractions run in FP32 on element-shifted fields, with the shifts added
-// back in FP64 -- exact in exact arithmetic because B reproduces constants
-// and the rows of D annihilate them:
+// Mixed-precision volume kernel (PM 1, 2): Gauss-point gradients into LDS
+// (Gauss_Deriv, SolnDerivsc.f90:14-83), then for each staggered grid the
+// interpolated state, prolonged gradients, contravariant Euler + viscous
+// fluxes, the viscous face traces r/norm and the interior part of the
+// divergence.  The LDS tiles hold FP32 values and the contractions run in
+// FP32 on element-shifted fields, with the shifts added back in FP64 --
+// exact in exact arithmetic because B reproduces constants and the rows of
+// D annihilate them:
 //   Q     - Qbar   (Qbar = Q at the element's central Gauss point);
 //   faces QA - Qbar in the gradient (D Qbar = 0 is dropped);
 //   flux  F - Fbar_d (Fbar_d = contravariant Euler flux of Qbar with the
 //         metric row at staggered point 0 of grid d); the divergence adds
 //         Fbar_d * sum_{interior j} D[k][j] back in FP64.
-// Pointwise physics, the gradient metric combination inputs, the RK state
-// and all face kernels stay FP64.
-// PLAIN: aligned faces, no entropy or eddy viscosity, no lagged states saved.
-// That instance compiles the optional paths out (at p = 8 FP64: 126 VGPRs
-// and no spill against 128 with a 12-byte spill, a quarter fewer VALU
-// instructions in the code); the other handles every case by run-time
-// branches.  The mixed modes use the general instance only: their plain one
-// spilled 28 bytes at p = 8 and ran slower.
-template <int P, int PM, bool PLAIN>
-__global__ __launch_bounds__((vblock<P, PM>()), 4) void k_volume(const double *__restrict__ JQ, DevMesh m, DevPhys ph,
-                                                    const double *__restrict__ QA, const double *__restrict__ muh,
-                                                    const double *__restrict__ nut, double *__restrict__ FV,
-                                                    double *__restrict__ Qtp, double *__restrict__ Slag)
+// Pointwise physics, the RK state and all face kernels stay FP64.
+template <int P, int PM>
+__global__ __launch_bounds__(VBLOCK, 4) void k_volume(const double *__restrict__ JQ, DevMesh m, DevPhys ph,
+                                                      const double *__restrict__ QA, const double *__restrict__ muh,
+                                                      const double *__restrict__ nut, double *__restrict__ FV,
+                                                      double *__restrict__ Qtp, double *__restrict__ Slag)
 {
-    if constexpr (PLAIN) {
-        muh = nullptr;
-        nut = nullptr;
-        Slag = nullptr;
-        m.rot = 0;
-    }
     using S = Sz<P>;
     using CT = typename Ctr<PM>::T;
     using CA = typename Ctr<PM>::A;
-    constexpr int VBLOCK = vblock<P, PM>();
     constexpr int R = (S::NP + VBLOCK - 1) / VBLOCK;
-    __shared__ CT sQ[NEQ * S::NP];            // physical Q at Gauss points (minus Qbar when mixed)
+    __shared__ CT sQ[NEQ * S::NP];            // physical Q at Gauss points minus Qbar
     __shared__ CT sG[15 * S::NP];             // dQ_v/dx_c at Gauss points, (c*5+v)
-    // interior total flux of the current grid (minus Fbar); during the
+    // interior total flux of the current grid minus Fbar; during the
     // gradient phase it holds the face averages of the six faces
     constexpr int NSF = NEQ * S::NS > 6 * NEQ * S::NF ? NEQ * S::NS : 6 * NEQ * S::NF;
     __shared__ CT sF[NSF];
-    __shared__ double sBar[5 + 15];           // mixed modes: Qbar[5], Fbar[3][5]
+    __shared__ double sBar[5 + 15];           // Qbar[5], Fbar[3][5]
     // operator matrices of this order: M = D_int B (Gauss derivative), D, B
     constexpr int OM = 0, OD = S::NCG * S::NCG, OB = OD + S::NCG * S::NC, NOP = OB + S::NC * S::NCG;
     __shared__ CT sOp[NOP];
-    __shared__ double sDint[S::NCG];          // mixed modes: sum over interior j of D[k][j]
-    const int tid0 = threadIdx.x;
-    constexpr bool MF = (PM == 0);
+    __shared__ double sDint[S::NCG];          // sum over interior j of D[k][j]
+    const int tid = threadIdx.x, e = blockIdx.x;
     constexpr int NQV = NEQ * S::NP, NAV = 6 * NEQ * S::NF;
     constexpr int NQI = (NQV + VBLOCK - 1) / VBLOCK, NAI = (NAV + VBLOCK - 1) / VBLOCK;
     constexpr int NOI = (NOP + VBLOCK - 1) / VBLOCK;
-    static_assert(NAV <= 15 * S::NP, "the face averages of the next element fit in sG");
-    // operator matrices, stored once per workgroup (the first element's
-    // barrier after its staging publishes them)
 #pragma unroll
     for (int u = 0; u < NOI; ++u) {
-        const int i = tid0 + u * VBLOCK;
-        if (i < NOP) {
-            const CT *src;
-            if constexpr (PM == 0) src = i < OD ? &c_M[P][i - OM] : (i < OB ? &c_D[P][i - OD] : &c_B[P][i - OB]);
-            else src = i < OD ? &c_Mf[P][i - OM] : (i < OB ? &c_Df[P][i - OD] : &c_Bf[P][i - OB]);
-            sOp[i] = *src;
-        }
+        const int i = tid + u * VBLOCK;
+        if (i < NOP) sOp[i] = i < OD ? c_Mf[P][i - OM] : (i < OB ? c_Df[P][i - OD] : c_Bf[P][i - OB]);
     }
-    // Persistent workgroup: elements blockIdx.x, + gridDim.x, ...  At 1024
-    // work-items (one workgroup per CU, nothing else to hide a memory wait)
-    // the FP64 form copies the next element's state, 1/J and face averages
-    // straight into sQ and sG (both free once the last grid's point pass is
-    // done) during the last divergence pass, so that only a workgroup's first
-    // element waits for its prologue.
-    constexpr bool PRE = MF && VBLOCK == 1024;
-    static_assert(!PRE || NAV + S::NP <= 15 * S::NP, "the next element's 1/J and face averages fit in sG");
-    // PRE: e2m entries of this element and of the next, in alternating slots
-    __shared__ int sE2m[2][6];
     const int npm = m.ms ? S::NP : 1;
-    if constexpr (PRE) {
-        // the workgroup's first element: its e2m entries and those of the
-        // next, then its inputs copied into LDS like every later element's
-        const int e0 = blockIdx.x, e1 = min(e0 + (int)gridDim.x, m.K - 1);
-        if (tid0 < 6) sE2m[0][tid0] = m.e2m[(size_t)e0 * 6 + tid0];
-        else if (tid0 < 12) sE2m[1][tid0 - 6] = m.e2m[(size_t)e1 * 6 + tid0 - 6];
-        __syncthreads();
-        volume_inputs_lds<P>(JQ, QA, m, e0, sE2m[0], tid0, sQ, sG + NAV, sG);
-    }
-    // Without PRE the body runs once (grid = elements) and there is no loop.
-    int slot = 0;
-    int e = blockIdx.x;
-#pragma unroll 1
-    while (true) {
-        const bool first = (e == blockIdx.x);
-        // The work-item index passes through an empty asm once per element:
-        // left visible, every index the element's passes derive from it (and
-        // the matrix-core operand fragments) is hoisted out of the loop and
-        // held in registers for its whole length (past 128 VGPRs, and into
-        // scratch, at 1024 work-items).
-        const int tid = PRE ? opaque(tid0) : tid0;
-        const MfLane<P> ml = mf_lane<P>(tid, c_B[P]);
-        const MfLane<P, S::NCG> mg = mf_lane<P, S::NCG>(tid, c_M[P]);   // gradient tiles (FP64 form)
-        CA gpre[R][9];
-        const double *jac = m.jacob + (size_t)e * (m.ms ? S::NP : 1);
-        const int nxt = e + gridDim.x;
-        int e2r[6];
-        const int *e2m_e = e2r;
-        if constexpr (PRE) {
-            e2m_e = sE2m[slot];
-        } else {
+    CA gpre[R][9];
+    const double *jac = m.jacob + (size_t)e * (m.ms ? S::NP : 1);
+    int e2m_e[6];
 #pragma unroll
-            for (int f = 0; f < 6; ++f) e2r[f] = m.e2m[(size_t)e * 6 + f];
-        }
-
-        // ---- prologue.  Every global load of the element's inputs is issued
-        // before the first wait: one exposed memory latency per element
-        // instead of one per loop trip.
-        double qv[NQI], jv[NQI], av[NAI];
-        if constexpr (!PRE) volume_inputs<P, PM>(JQ, QA, m, e, tid, qv, jv, av);
-        // the previous element is done with sQ, sG, sF; PRE: this element's
-        // copies into LDS have landed
-        if constexpr (PRE) lds_copies_done();
-        if (PRE || !first) __syncthreads();
-        {
-            // metric rows of this work-item's Gauss points, first used after
-            // the gradient contractions
-            const double *gg = m.gmetg + (size_t)e * 9 * npm;
-#pragma unroll
-            for (int r = 0; r < R; ++r) {
-                const int pt = tid + r * VBLOCK;
-                if constexpr (PM != 0) {
-                    // mixed modes: unconditional loads from a clamped point,
-                    // converted after the select (guarded, converting loads:
-                    // 1.11 ms at 22^3 p=8 FP32, these: 0.98 ms; the FP64
-                    // kernel is faster with the guarded form)
-                    const int pc = pt < S::NP ? pt : S::NP - 1;
-#pragma unroll
-                    for (int i = 0; i < 9; ++i) {
-                        const double g = gg[i * npm + pc * m.ms];
-                        gpre[r][i] = (CA)(pt < S::NP ? g : 0.0);
-                    }
-                } else {
-#pragma unroll
-                    for (int i = 0; i < 9; ++i) gpre[r][i] = pt < S::NP ? (CA)gg[i * npm + pt * m.ms] : (CA)0;
-                }
-            }
-        }
-        if constexpr (PM != 0) {
-            // Qbar = Q at the central Gauss point, Fbar_d = Euler flux of Qbar
-            // with the metric row at staggered point 0 of grid d
-            constexpr int pc = (S::NCG / 2) * (1 + S::NCG + S::NCG * S::NCG);
-            const int nsm = m.ms ? S::NS : 1;
-            double qc = 0.0, gm[3] = {0.0, 0.0, 0.0};
-            if (tid < 5) qc = JQ[((size_t)e * NEQ + tid) * S::NP + pc] * jac[pc * m.ms];
-            if (tid < 3) {
-                const double *gmd = (tid == 0 ? m.gmet0 : (tid == 1 ? m.gmet1 : m.gmet2)) + (size_t)e * 3 * nsm;
-#pragma unroll
-                for (int i = 0; i < 3; ++i) gm[i] = gmd[i * nsm];
-            }
-            if (tid < S::NCG) sDint[tid] = c_Dint[P][tid];
-            if (tid < 5) sBar[tid] = qc;
-            __syncthreads();
-            if (tid < 3) {
-                double qb[5], fb[5];
-#pragma unroll
-                for (int v = 0; v < 5; ++v) qb[v] = sBar[v];
-                const Prim pb = primitives(ph, qb);
-                euler_from_primitive(pb, qb, gm[0], gm[1], gm[2], fb);
-#pragma unroll
-                for (int v = 0; v < 5; ++v) sBar[5 + tid * 5 + v] = fb[v];
-            }
-        }
-
-        CT *sQA = sF;   // face averages of the six faces (face f+1 at [f][v][q]), minus Qbar when mixed
-        if constexpr (PRE) {
-            // sQ holds this element's raw J*Q, sG its face averages and (from
-            // NAV on) 1/J: Q = (J*Q) (1/J) in place
-            for (int i = tid; i < NQV; i += VBLOCK) sQ[i] = sQ[i] * sG[NAV + i % S::NP];
-            for (int i = tid; i < NAV; i += VBLOCK) sQA[i] = sG[i];
-        } else {
-#pragma unroll
-            for (int u = 0; u < NQI; ++u) {
-                const int i = tid + u * VBLOCK;
-                if (i < NQV) {
-                    const double qp = qv[u] * jv[u];
-                    if constexpr (PM == 0) sQ[i] = qp; else sQ[i] = (CT)(qp - sBar[i / S::NP]);
-                }
-            }
-#pragma unroll
-            for (int u = 0; u < NAI; ++u) {
-                const int i = tid + u * VBLOCK;
-                if (i < NAV) {
-                    if constexpr (PM == 0) sQA[i] = av[u]; else sQA[i] = (CT)(av[u] - sBar[(i % (NEQ * S::NF)) / S::NF]);
-                }
-            }
-        }
-        __syncthreads();
-
-        // ---- gradients: w_d = (D_int B) Q + D(:,0) QA_lo + D(:,nc-1) QA_hi, then metric combine
-        if constexpr (MF) {
-            // Matrix-core form.  Direction by direction, the tile lane of each
-            // Gauss point writes w_d (5 fields) into slots d*5+v of sG; one
-            // direction's tiles cover every point once, so the three directions
-            // need no barrier between them.  Then each work-item combines the 15
-            // w values of its point with the metric rows, in place, in the same
-            // order as the vector form: g0 w0, then + g1 w1, then + g2 w2.
-            constexpr int KSG = MfTiles<P, S::NCG>::KS;
-            static_assert(MfTiles<P, S::NCG>::NT <= VBLOCK / 16, "one gradient tile per 16 lanes in one pass");
-            if (mg.wave_active) {
-                const int a = mg.line % S::NCG, b = mg.line / S::NCG;   // mg.line = a + ncg b
-#pragma unroll
-                for (int d = 0; d < 3; ++d) {
-                    int off[KSG];
-#pragma unroll
-                    for (int ks = 0; ks < KSG; ++ks) {
-                        const int k = 4 * ks + mg.r;
-                        off[ks] = gidx<P>(d, k < S::NCG ? k : S::NCG - 1, a, b);
-                    }
-                    double w[5];
-#pragma unroll
-                    for (int v = 0; v < 5; ++v) w[v] = mf_line<P, S::NCG>(sQ + v * S::NP, mg, off);
-                    if (mg.valid) {
-                        const int k = mg.j;
-                        const double d0 = sOp[OD + k * S::NC], d1 = sOp[OD + k * S::NC + S::NC - 1];
-                        const double *qa0 = sQA + (face_of<P>(d, 0) - 1) * NEQ * S::NF + mg.line;
-                        const double *qa1 = sQA + (face_of<P>(d, 1) - 1) * NEQ * S::NF + mg.line;
-                        const int pt = gidx<P>(d, k, a, b);
-#pragma unroll
-                        for (int v = 0; v < 5; ++v)
-                            sG[(d * 5 + v) * S::NP + pt] = fma(d1, qa1[v * S::NF], fma(d0, qa0[v * S::NF], w[v]));
-                    }
-                }
-            }
-            __syncthreads();
-#pragma unroll
-            for (int r = 0; r < R; ++r) {
-                const int pt = tid + r * VBLOCK;
-                if (pt >= S::NP) break;
-                double w[15];
-#pragma unroll
-                for (int i = 0; i < 15; ++i) w[i] = sG[i * S::NP + pt];
-                const CA *g = gpre[r];
-#pragma unroll
-                for (int c = 0; c < 3; ++c)
-#pragma unroll
-                    for (int v = 0; v < 5; ++v)
-                        sG[(c * 5 + v) * S::NP + pt] = fma(g[6 + c], w[10 + v], fma(g[3 + c], w[5 + v], g[c] * w[v]));
-            }
-        } else {
-#pragma unroll
-            for (int r = 0; r < R; ++r) {
-                const int pt = tid + r * VBLOCK;
-                if (pt >= S::NP) break;
-                const int n = pt % S::NCG, mi = (pt / S::NCG) % S::NCG, l = pt / (S::NCG * S::NCG);
-                CA out[3][5];
-#pragma unroll
-                for (int d = 0; d < 3; ++d) {
-                    const int k = d == 0 ? n : (d == 1 ? mi : l);
-                    const int a = d == 0 ? mi : n;
-                    const int b = d == 2 ? mi : l;
-                    const int q = a + S::NCG * b;
-                    CT Mk[S::NCG];
-#pragma unroll
-                    for (int k2 = 0; k2 < S::NCG; ++k2) Mk[k2] = sOp[OM + k * S::NCG + k2];
-                    const CT d0 = sOp[OD + k * S::NC], d1 = sOp[OD + k * S::NC + S::NC - 1];
-                    const CT *qa0 = sQA + (face_of<P>(d, 0) - 1) * NEQ * S::NF + q;
-                    const CT *qa1 = sQA + (face_of<P>(d, 1) - 1) * NEQ * S::NF + q;
-                    const CA *gd = gpre[r] + d * 3;
-#pragma unroll
-                    for (int v = 0; v < 5; ++v) {
-                        CA t = 0;
-#pragma unroll
-                        for (int k2 = 0; k2 < S::NCG; ++k2) t = mac<PM>(Mk[k2], sQ[v * S::NP + gidx<P>(d, k2, a, b)], t);
-                        t = mac<PM>(d0, qa0[v * S::NF], t);
-                        t = mac<PM>(d1, qa1[v * S::NF], t);
-#pragma unroll
-                        for (int c = 0; c < 3; ++c) out[c][v] = d == 0 ? gd[c] * t : fma(gd[c], t, out[c][v]);
-                    }
-                    __builtin_amdgcn_sched_barrier(0);
-                }
-#pragma unroll
-                for (int c = 0; c < 3; ++c)
-#pragma unroll
-                    for (int v = 0; v < 5; ++v) sG[(c * 5 + v) * S::NP + pt] = (CT)out[c][v];
-            }
-        }
-
-
-        double acc[R][5];
-#pragma unroll
-        for (int r = 0; r < R; ++r)
-#pragma unroll
-            for (int v = 0; v < 5; ++v) acc[r][v] = 0.0;
-        LaneFlux lf;
-        lf = volume_grid<P, 0, PM, MF>(m, ph, QA, muh, nut, FV, Slag, sQ, sG, sF, sBar, sOp + OD, sOp + OB, sDint, e, e2m_e, ml, tid);
-        volume_publish<P, 0, PM, MF>(lf, sF);
-        volume_div<P, 0, PM>(sF, sOp + OD, sBar, sDint, tid, acc);
-        lf = volume_grid<P, 1, PM, MF>(m, ph, QA, muh, nut, FV, Slag, sQ, sG, sF, sBar, sOp + OD, sOp + OB, sDint, e, e2m_e, ml, tid);
-        volume_publish<P, 1, PM, MF>(lf, sF);
-        volume_div<P, 1, PM>(sF, sOp + OD, sBar, sDint, tid, acc);
-        lf = volume_grid<P, 2, PM, MF>(m, ph, QA, muh, nut, FV, Slag, sQ, sG, sF, sBar, sOp + OD, sOp + OB, sDint, e, e2m_e, ml, tid);
-        volume_publish<P, 2, PM, MF>(lf, sF);
-        if constexpr (PRE) {
-            // wait for this element's face-trace stores first, in a form the
-            // compiler accounts for (on every path): a wait it placed later
-            // for them would also wait for every copy issued after them
-            __builtin_amdgcn_s_waitcnt(VMCNT0);
-            if (nxt < m.K) {
-                // every wave is past this element's point passes: the next
-                // element's inputs go into sQ and sG, and the e2m entries of
-                // the element after it into the slot this element is done with
-                const int *e2m_n = sE2m[slot ^ 1];
-                volume_inputs_lds<P>(JQ, QA, m, nxt, e2m_n, tid, sQ, sG + NAV, sG);
-                const int n2 = min(nxt + (int)gridDim.x, m.K - 1);
-                if (tid < 6) lds_dword(m.e2m + (size_t)n2 * 6 + tid, sE2m[slot]);
-            }
-        }
-        volume_div<P, 2, PM>(sF, sOp + OD, sBar, sDint, tid, acc);
+    for (int f = 0; f < 6; ++f) e2m_e[f] = m.e2m[(size_t)e * 6 + f];
+    // ---- prologue.  Every global load of the element's inputs is issued
+    // before the first wait: one exposed memory latency per element instead
+    // of one per loop trip.
+    double qv[NQI], jv[NQI], av[NAI];
+    volume_inputs<P>(JQ, QA, m, e, tid, qv, jv, av);
+    {
+        // metric rows of this work-item's Gauss points, first used after the
+        // gradient contractions: unconditional loads from a clamped point,
+        // converted after the select (guarded, converting loads: 1.11 ms at
+        // 22^3 p=8 FP32, these: 0.98 ms)
+        const double *gg = m.gmetg + (size_t)e * 9 * npm;
 #pragma unroll
         for (int r = 0; r < R; ++r) {
             const int pt = tid + r * VBLOCK;
-            if (pt < S::NP)
+            const int pc = pt < S::NP ? pt : S::NP - 1;
 #pragma unroll
-                for (int v = 0; v < 5; ++v) Qtp[((size_t)e * NEQ + v) * S::NP + pt] = acc[r][v];
+            for (int i = 0; i < 9; ++i) {
+                const double g = gg[i * npm + pc * m.ms];
+                gpre[r][i] = (CA)(pt < S::NP ? g : 0.0);
+            }
         }
-        if constexpr (!PRE) break;
-        e += gridDim.x;
-        slot ^= 1;
-        if (e >= m.K) break;
+    }
+    {
+        // Qbar = Q at the central Gauss point, Fbar_d = Euler flux of Qbar
+        // with the metric row at staggered point 0 of grid d
+        constexpr int pc = (S::NCG / 2) * (1 + S::NCG + S::NCG * S::NCG);
+        const int nsm = m.ms ? S::NS : 1;
+        double qc = 0.0, gm[3] = {0.0, 0.0, 0.0};
+        if (tid < 5) qc = JQ[((size_t)e * NEQ + tid) * S::NP + pc] * jac[pc * m.ms];
+        if (tid < 3) {
+            const double *gmd = m.gmet + ((size_t)e * 3 + tid) * 3 * nsm;
+#pragma unroll
+            for (int i = 0; i < 3; ++i) gm[i] = gmd[i * nsm];
+        }
+        if (tid < S::NCG) sDint[tid] = c_Dint[P][tid];
+        if (tid < 5) sBar[tid] = qc;
+        __syncthreads();
+        if (tid < 3) {
+            double qb[5], fb[5];
+#pragma unroll
+            for (int v = 0; v < 5; ++v) qb[v] = sBar[v];
+            const Prim pb = primitives(ph, qb);
+            euler_from_primitive(pb, qb, gm[0], gm[1], gm[2], fb);
+#pragma unroll
+            for (int v = 0; v < 5; ++v) sBar[5 + tid * 5 + v] = fb[v];
+        }
+    }
+    CT *sQA = sF;   // face averages of the six faces minus Qbar (face f+1 at [f][v][q])
+#pragma unroll
+    for (int u = 0; u < NQI; ++u) {
+        const int i = tid + u * VBLOCK;
+        if (i < NQV) sQ[i] = (CT)(qv[u] * jv[u] - sBar[i / S::NP]);
+    }
+#pragma unroll
+    for (int u = 0; u < NAI; ++u) {
+        const int i = tid + u * VBLOCK;
+        if (i < NAV) sQA[i] = (CT)(av[u] - sBar[(i % (NEQ * S::NF)) / S::NF]);
+    }
+    __syncthreads();
+
+    // ---- gradients: w_d = (D_int B) Q + D(:,0) QA_lo + D(:,nc-1) QA_hi, then metric combine
+#pragma unroll
+    for (int r = 0; r < R; ++r) {
+        const int pt = tid + r * VBLOCK;
+        if (pt >= S::NP) break;
+        const int n = pt % S::NCG, mi = (pt / S::NCG) % S::NCG, l = pt / (S::NCG * S::NCG);
+        CA out[3][5];
+#pragma unroll
+        for (int d = 0; d < 3; ++d) {
+            const int k = d == 0 ? n : (d == 1 ? mi : l);
+            const int a = d == 0 ? mi : n;
+            const int b = d == 2 ? mi : l;
+            const int q = a + S::NCG * b;
+            CT Mk[S::NCG];
+#pragma unroll
+            for (int k2 = 0; k2 < S::NCG; ++k2) Mk[k2] = sOp[OM + k * S::NCG + k2];
+            const CT d0 = sOp[OD + k * S::NC], d1 = sOp[OD + k * S::NC + S::NC - 1];
+            const CT *qa0 = sQA + (face_of<P>(d, 0) - 1) * NEQ * S::NF + q;
+            const CT *qa1 = sQA + (face_of<P>(d, 1) - 1) * NEQ * S::NF + q;
+            const CA *gd = gpre[r] + d * 3;
+#pragma unroll
+            for (int v = 0; v < 5; ++v) {
+                CA t = 0;
+#pragma unroll
+                for (int k2 = 0; k2 < S::NCG; ++k2) t = mac<PM>(Mk[k2], sQ[v * S::NP + gidx<P>(d, k2, a, b)], t);
+                t = mac<PM>(d0, qa0[v * S::NF], t);
+                t = mac<PM>(d1, qa1[v * S::NF], t);
+#pragma unroll
+                for (int c = 0; c < 3; ++c) out[c][v] = d == 0 ? gd[c] * t : fma(gd[c], t, out[c][v]);
+            }
+            __builtin_amdgcn_sched_barrier(0);
+        }
+#pragma unroll
+        for (int c = 0; c < 3; ++c)
+#pragma unroll
+            for (int v = 0; v < 5; ++v) sG[(c * 5 + v) * S::NP + pt] = (CT)out[c][v];
+    }
+
+    double acc[R][5];
+#pragma unroll
+    for (int r = 0; r < R; ++r)
+#pragma unroll
+        for (int v = 0; v < 5; ++v) acc[r][v] = 0.0;
+    volume_grid<P, 0, PM>(m, ph, QA, muh, nut, FV, Slag, sQ, sG, sF, sBar, sOp + OB, e, e2m_e, tid);
+    volume_div<P, 0, PM>(sF, sOp + OD, sBar, sDint, tid, acc);
+    volume_grid<P, 1, PM>(m, ph, QA, muh, nut, FV, Slag, sQ, sG, sF, sBar, sOp + OB, e, e2m_e, tid);
+    volume_div<P, 1, PM>(sF, sOp + OD, sBar, sDint, tid, acc);
+    volume_grid<P, 2, PM>(m, ph, QA, muh, nut, FV, Slag, sQ, sG, sF, sBar, sOp + OB, e, e2m_e, tid);
+    volume_div<P, 2, PM>(sF, sOp + OD, sBar, sDint, tid, acc);
+#pragma unroll
+    for (int r = 0; r < R; ++r) {
+        const int pt = tid + r * VBLOCK;
+        if (pt < S::NP)
+#pragma unroll
+            for (int v = 0; v < 5; ++v) Qtp[((size_t)e * NEQ + v) * S::NP + pt] = acc[r][v];
     }
 }
+
+#include "volume.inc"
 
 template <int P>
 __global__ __launch_bounds__(BLOCK) void k_face_visc(const double *__restrict__ FV, const double *__restrict__ FI,
@@ -1923,7 +1579,7 @@ __global__ __launch_bounds__(BLOCK) void k_dtcalc(const double *__restrict__ JQ,
         const int s0 = (n + S::NC * (mi + S::NCG * l)) * m.ms;
         const int s1 = (n + S::NCG * (mi + S::NC * l)) * m.ms;
         const int s2 = (n + S::NCG * (mi + S::NCG * l)) * m.ms;
-        const double *g0 = m.gmet0 + (size_t)e * 3 * nsm, *g1 = m.gmet1 + (size_t)e * 3 * nsm, *g2 = m.gmet2 + (size_t)e * 3 * nsm;
+        const double *g0 = m.gmet + (size_t)e * 9 * nsm, *g1 = g0 + 3 * nsm, *g2 = g1 + 3 * nsm;
         const double uu = (u0 + a) * g0[s0] + (v0 + a) * g0[nsm + s0] + (w0 + a) * g0[2 * nsm + s0];
         const double vv = (u0 + a) * g1[s1] + (v0 + a) * g1[nsm + s1] + (w0 + a) * g1[2 * nsm + s1];
         const double ww = (u0 + a) * g2[s2] + (v0 + a) * g2[nsm + s2] + (w0 + a) * g2[2 * nsm + s2];
@@ -2041,19 +1697,19 @@ struct dsem_ctx {
     std::string err;
     hipStream_t stream = nullptr;
     dsem::Ops ops;
-    std::vector<double> h_xg, h_jacob;   // Gauss points and 1/J on the host
+    dsem::Array h_xg, h_jacob;           // Gauss points and 1/J on the host
     std::vector<double> h_corners;       // [K][8][3], for host-side geometry queries
     std::vector<int32_t> h_melem, h_mface;
     // device buffers
     double *JQ = nullptr, *G = nullptr, *Qtp = nullptr, *Qt = nullptr;
     double *T = nullptr, *FV = nullptr, *QA = nullptr, *FI = nullptr, *FT = nullptr;
-    double *jacob = nullptr, *gmetg = nullptr, *gmet[3] = {nullptr, nullptr, nullptr};
+    double *jacob = nullptr, *gmetg = nullptr, *gmet = nullptr;
     double *nhat = nullptr, *norm = nullptr, *muh = nullptr;
     double *Slag = nullptr, *muhg = nullptr, *ev_resid = nullptr, *ev_ducros = nullptr;   // entropy viscosity
     bool have_lag = false;
     bool keep_lag = false;                     // save the last stage's staggered states without EV
     bool traces_cur = false;                   // T holds the face traces of the current JQ
-    int vol_grid[3] = {0, 0, 0};               // resident volume-kernel workgroups per precision mode
+    int vol_grid = 0;                          // resident workgroups of the persistent FP64 volume kernel
     bool les = false;                          // static Smagorinsky model
     double les_cs = 0.0, les_numax = 0.0;
     double *nut = nullptr, *nut_g = nullptr;   // eddy viscosity on the staggered grids / Gauss points
@@ -2116,8 +1772,8 @@ int dev_alloc(dsem_ctx *c, T **p, size_t n)
     return DSEM_OK;
 }
 
-template <typename T>
-int upload(dsem_ctx *c, T **p, const std::vector<T> &h)
+template <typename T, typename A>
+int upload(dsem_ctx *c, T **p, const std::vector<T, A> &h)
 {
     int rc = dev_alloc(c, p, h.size());
     if (rc) return rc;
@@ -2129,7 +1785,7 @@ DevMesh dev_mesh(const dsem_ctx *c)
 {
     DevMesh m;
     m.K = c->K; m.M = c->M; m.ms = c->ms;
-    m.jacob = c->jacob; m.gmetg = c->gmetg; m.gmet0 = c->gmet[0]; m.gmet1 = c->gmet[1]; m.gmet2 = c->gmet[2];
+    m.jacob = c->jacob; m.gmetg = c->gmetg; m.gmet = c->gmet;
     m.e2m = c->e2m; m.m_elem = c->m_elem; m.m_face = c->m_face; m.m_sign = c->m_sign; m.m_nsign = c->m_nsign;
     m.m_orient = c->m_orient;
     m.rot = c->rotated ? 1 : 0;
@@ -2177,35 +1833,28 @@ int launch(dsem_ctx *c, int kid, F &&fn)
         if (rc_) return rc_;   \
     } while (0)
 
-// Workgroups of the volume kernel.  The FP64 kernels of 1024 work-items
-// (p >= 7) are persistent: as many workgroups as are resident at once, each
-// looping over elements with a stride of the grid (never more than the
-// elements; queried once per context).  The others take one element each.
-template <int P, int PM>
+// Workgroups of the FP64 volume kernel.  k_volume_mf is persistent: as many
+// workgroups as are resident at once, each looping over elements with a
+// stride of the grid (never more than the elements; queried once per
+// context).  In k_volume_vec each workgroup takes one element.
+template <int P>
 int volume_grid_size(dsem_ctx *c, int &grid)
 {
-    if (!(PM == 0 && vblock<P, PM>() == 1024)) {
-        grid = c->K;
-        return DSEM_OK;
+    grid = c->K;
+    if constexpr (Vol<P>::MF) {
+        int &g = c->vol_grid;
+        if (g == 0) {
+            int per_cu = 0, ncu = 0;
+            HIP_TRY(c, hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, k_volume_mf<P, 3, true>, Vol<P>::BLK, 0));
+            HIP_TRY(c, hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, c->device));
+            if (per_cu < 1 || ncu < 1) return set_err(c, DSEM_ERR_HIP, "volume kernel: no resident work-group fits");
+            g = per_cu * ncu;
+        }
+        grid = g < c->K ? g : c->K;
     }
-    int &g = c->vol_grid[PM];
-    if (g == 0) {
-        int per_cu = 0, ncu = 0;
-        // both instances hold the same LDS, which allows one workgroup per CU
-        HIP_TRY(c, hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, k_volume<P, PM, false>, vblock<P, PM>(), 0));
-        HIP_TRY(c, hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, c->device));
-        if (per_cu < 1 || ncu < 1) return set_err(c, DSEM_ERR_HIP, "volume kernel: no resident work-group fits");
-        g = per_cu * ncu;
-    }
-    grid = g < c->K ? g : c->K;
     return DSEM_OK;
 }
 
-// One RHS evaluation on state JQ; the final kernel either writes Qt or
-// performs an RK register update (st.rk).
-// traces_ready: T already holds the face traces of JQ (computed by the
-// previous stage's update); make_traces: this stage's update also computes
-// the traces of the updated state for the next stage.
 // Per-call intermediates of one RHS evaluation: face traces T, mortar
 // averages QA, Roe fluxes FI, viscous face traces FV, total face fluxes FT
 // and the partial residual Qtp.  Every entry a call reads is written earlier
@@ -2216,6 +1865,34 @@ struct RhsBufs {
 
 RhsBufs ctx_bufs(const dsem_ctx *c) { return RhsBufs{c->T, c->QA, c->FI, c->FV, c->FT, c->Qtp}; }
 
+// The instance of the FP64 volume kernel for this call's viscosities.
+template <int P>
+void run_volume64(dsem_ctx *c, const double *JQ, const DevMesh &m, const DevPhys &ph, const RhsBufs &b,
+                  const double *muh, const double *nut, double *slag, int grid)
+{
+    auto go = [&](auto model, auto lag) {
+        constexpr int MODEL = decltype(model)::value;
+        constexpr bool LAG = decltype(lag)::value;
+        if constexpr (Vol<P>::MF)
+            k_volume_mf<P, MODEL, LAG><<<grid, Vol<P>::BLK, 0, c->stream>>>(JQ, m, ph, b.QA, muh, nut, b.FV, b.Qtp, slag);
+        else
+            k_volume_vec<P, MODEL, LAG><<<grid, Vol<P>::BLK, 0, c->stream>>>(JQ, m, ph, b.QA, muh, nut, b.FV, b.Qtp, slag);
+    };
+    auto lagged = [&](auto model) {
+        if (slag) go(model, std::true_type{});
+        else go(model, std::false_type{});
+    };
+    if (nut && muh) lagged(std::integral_constant<int, 3>{});
+    else if (nut) lagged(std::integral_constant<int, 2>{});
+    else if (muh) lagged(std::integral_constant<int, 1>{});
+    else lagged(std::integral_constant<int, 0>{});
+}
+
+// One RHS evaluation on state JQ; the final kernel either writes Qt or
+// performs an RK register update (st.rk).
+// traces_ready: T already holds the face traces of JQ (computed by the
+// previous stage's update); make_traces: this stage's update also computes
+// the traces of the updated state for the next stage.
 template <int P>
 int run_rhs(dsem_ctx *c, double *JQ, const StageArgs &st, double *Qt_out, bool traces_ready, bool make_traces,
             bool save_lag, const RhsBufs &b)
@@ -2232,25 +1909,15 @@ int run_rhs(dsem_ctx *c, double *JQ, const StageArgs &st, double *Qt_out, bool t
     if (!traces_ready) TRY(launch(c, KID_TRACES, [&] { k_traces<P><<<K, BLOCK, 0, s>>>(JQ, m, b.T); }));
     TRY(launch(c, KID_FACE_INV, [&] { k_face_inv<P><<<face_blocks, BLOCK, 0, s>>>(b.T, m, ph, b.FI, b.QA); }));
     double *slag = save_lag ? c->Slag : nullptr;
-    int gv0 = 0, gv1 = 0, gv2 = 0;
-    if (c->params.precision == DSEM_PREC_FP32) TRY((volume_grid_size<P, 1>(c, gv1)));
-    else if (c->params.precision == DSEM_PREC_BF16X3) TRY((volume_grid_size<P, 2>(c, gv2)));
-    else TRY((volume_grid_size<P, 0>(c, gv0)));
-    const bool plain = !c->rotated && !muh && !nut && !slag;
-    auto vol = [&](auto pm, auto pl, int grid) {
-        constexpr int PM = decltype(pm)::value;
-        k_volume<P, PM, decltype(pl)::value><<<grid, vblock<P, PM>(), 0, s>>>(JQ, m, ph, b.QA, muh, nut, b.FV, b.Qtp,
-                                                                             slag);
-    };
-    using T_ = std::true_type;
-    using F_ = std::false_type;
+    int grid = K;
+    if (c->params.precision == DSEM_PREC_FP64) TRY(volume_grid_size<P>(c, grid));
     TRY(launch(c, KID_VOLUME, [&] {
         if (c->params.precision == DSEM_PREC_FP32)
-            vol(std::integral_constant<int, 1>{}, F_{}, gv1);
+            k_volume<P, 1><<<K, VBLOCK, 0, s>>>(JQ, m, ph, b.QA, muh, nut, b.FV, b.Qtp, slag);
         else if (c->params.precision == DSEM_PREC_BF16X3)
-            vol(std::integral_constant<int, 2>{}, F_{}, gv2);
+            k_volume<P, 2><<<K, VBLOCK, 0, s>>>(JQ, m, ph, b.QA, muh, nut, b.FV, b.Qtp, slag);
         else
-            plain ? vol(std::integral_constant<int, 0>{}, T_{}, gv0) : vol(std::integral_constant<int, 0>{}, F_{}, gv0);
+            run_volume64<P>(c, JQ, m, ph, b, muh, nut, slag, grid);
     }));
     TRY(launch(c, KID_FACE_VISC, [&] { k_face_visc<P><<<face_blocks, BLOCK, 0, s>>>(b.FV, b.FI, m, ph, b.FT); }));
     if (make_traces)
@@ -2720,6 +2387,82 @@ int vjp_recorded_step(dsem_ctx *c, double dt, int slot, double *dQbar, double *n
     return DSEM_OK;
 }
 
+// Even-odd operators of one order (layout and reflections: volume.inc).  The
+// computed B, D and M obey the reflections up to rounding; each entry is the
+// mean of itself and its mirror image.
+template <int P>
+void even_odd_ops(const dsem::Ops &o, double *t)
+{
+    constexpr int n = P + 1, nc = P + 2, hg = n / 2, j0 = eo_first(P), nrw = Vol<P>::NRW;
+    auto B = [&](int j, int k) { return 0.5 * (o.B[j * n + k] + o.B[(nc - 1 - j) * n + n - 1 - k]); };
+    auto D = [&](int k, int j) { return 0.5 * (o.D[k * nc + j] - o.D[(n - 1 - k) * nc + nc - 1 - j]); };
+    auto M = [&](int k, int k2) { return 0.5 * (o.M[k * n + k2] - o.M[(n - 1 - k) * n + n - 1 - k2]); };
+    std::fill(t, t + EO_N, 0.0);
+    if constexpr (!Vol<P>::MF) return;
+    constexpr int slots = Vol<P>::MIDV ? hg : (n + 1) / 2;   // Gauss pairs that have a slot
+    for (int k = 0; k < slots; ++k) {
+        const int kr = n - 1 - k;
+        const double half = k == kr ? 0.25 : 0.5;   // the middle point meets itself: e = 2 x
+        for (int r = 0; r < nrw; ++r) {
+            t[EO_IE + r * 4 + k] = half * (B(j0 + r, k) + B(j0 + r, kr));
+            t[EO_IO + r * 4 + k] = 0.5 * (B(j0 + r, k) - B(j0 + r, kr));
+        }
+        for (int r = 0; r < slots; ++r) {
+            t[EO_GP + r * 4 + k] = half * (M(r, k) + M(r, kr));
+            t[EO_GR + r * 4 + k] = 0.5 * (M(r, k) - M(r, kr));
+        }
+        t[EO_GPF + k] = 0.5 * (D(k, 0) + D(k, nc - 1));
+        t[EO_GRF + k] = 0.5 * (D(k, 0) - D(k, nc - 1));
+    }
+    for (int r = 0; r < nrw; ++r) {
+        const int j = j0 + r, jr = nc - 1 - j;
+        if (j < 1) continue;                        // the face part of the divergence is k_update's
+        const double half = j == jr ? 0.25 : 0.5;
+        for (int k = 0; k < slots; ++k) {
+            t[EO_DP + k * 4 + r] = -half * (D(k, j) + D(k, jr));
+            t[EO_DR + k * 4 + r] = -0.5 * (D(k, j) - D(k, jr));
+        }
+    }
+    if constexpr (Vol<P>::MIDV) {
+        for (int r = 0; r < 4; ++r) {
+            t[EO_IM + r] = B(j0 + r, hg);
+            t[EO_DM + r] = -0.5 * (D(hg, j0 + r) - D(hg, nc - 1 - j0 - r));
+            t[EO_GPM + r] = M(r, hg);
+            t[EO_GM + r] = 0.5 * (M(hg, r) - M(hg, n - 1 - r));
+        }
+        t[EO_GMF] = 0.5 * (D(hg, 0) - D(hg, nc - 1));
+    }
+    // row sums of the reference operators minus those of the tiles: a
+    // constant field c enters the even part as 2 c and the odd part as 0
+    auto even_sum = [&](int tile, int row) {
+        long double s = 0.0L;
+        for (int k = 0; k < 4; ++k) s += 2.0L * t[tile + row * 4 + k];
+        return s;
+    };
+    for (int r = 0; r < nrw; ++r) {
+        const int j = j0 + r;
+        long double lo = 0.0L, hi = 0.0L;
+        for (int k = 0; k < n; ++k) {
+            lo += o.B[j * n + k];
+            hi += o.B[(nc - 1 - j) * n + k];
+        }
+        const long double s = even_sum(EO_IE, r) + (long double)t[EO_IM + r];
+        t[EO_CI + r] = (double)(lo - s);
+        t[EO_CI + 4 + r] = (double)(hi - s);
+    }
+    auto div_sum = [&](int k) {
+        long double s = 0.0L;
+        for (int j = 1; j <= P; ++j) s -= o.D[k * nc + j];
+        return s;
+    };
+    for (int k = 0; k < slots; ++k) {
+        const long double s = even_sum(EO_DP, k);
+        t[EO_CD + k] = (double)(div_sum(k) - s);
+        t[EO_CD + 4 + k] = (double)(div_sum(n - 1 - k) + s);   // row ncg-1-k is R - P
+    }
+    if constexpr (Vol<P>::MIDV) t[EO_CDM] = (double)div_sum(hg);
+}
+
 int upload_operators(dsem_ctx *c)
 {
     double D[9][90] = {}, B[9][90] = {}, Mo[9][81] = {}, cx[9][10] = {};
@@ -2751,6 +2494,19 @@ int upload_operators(dsem_ctx *c)
     HIP_TRY(c, hipMemcpyToSymbol(HIP_SYMBOL(c_Bf), Bf, sizeof(Bf)));
     HIP_TRY(c, hipMemcpyToSymbol(HIP_SYMBOL(c_Mf), Mf, sizeof(Mf)));
     HIP_TRY(c, hipMemcpyToSymbol(HIP_SYMBOL(c_Dint), Dint, sizeof(Dint)));
+    double eo[9][EO_N] = {};
+    {
+        dsem::Ops o;
+        auto fill = [&](auto p) {
+            dsem::make_ops(decltype(p)::value, o);
+            even_odd_ops<decltype(p)::value>(o, eo[decltype(p)::value]);
+        };
+        fill(std::integral_constant<int, 5>{});
+        fill(std::integral_constant<int, 6>{});
+        fill(std::integral_constant<int, 7>{});
+        fill(std::integral_constant<int, 8>{});
+    }
+    HIP_TRY(c, hipMemcpyToSymbol(HIP_SYMBOL(c_eo), eo, sizeof(eo)));
     double C2[9][81] = {}, C3[9][81] = {};
     const double pi = 3.141592653589793238462643;
     for (int p = 1; p <= 8; ++p) {
@@ -2840,34 +2596,35 @@ int create_impl(const dsem_mesh_desc *mesh, const dsem_params *prm, int device, 
 
     dsem::Geometry g;
     dsem::element_geometry(c->ops, c->K, mesh->corners, g);
-    std::vector<double> nhat, norm;
+    dsem::Array nhat, norm;
     dsem::mortar_geometry(c->ops, c->M, mesh->corners, mesh->mortar_elem, mesh->mortar_face, nhat, norm);
-    c->h_xg = g.xg;
+    c->h_xg = std::move(g.xg);
     c->h_corners.assign(mesh->corners, mesh->corners + (size_t)c->K * 24);
     c->h_melem.assign(mesh->mortar_elem, mesh->mortar_elem + 2 * (size_t)c->M);
     c->h_mface.assign(mesh->mortar_face, mesh->mortar_face + 2 * (size_t)c->M);
-    c->h_jacob = g.jacob;
     int mode = prm->metrics;
     if (mode == DSEM_METRICS_AUTO) mode = g.affine ? DSEM_METRICS_PER_ELEMENT : DSEM_METRICS_PER_POINT;
     if (mode == DSEM_METRICS_PER_ELEMENT && !g.affine)
         return set_err(c, DSEM_ERR_ARG, "per-element metrics need parallelepiped elements");
     c->ms = (mode == DSEM_METRICS_PER_ELEMENT) ? 0 : 1;
     if (c->ms == 0) {
+        c->h_jacob = g.jacob;
         // keep the value at the first point of every element / mortar
-        auto compact = [](std::vector<double> &v, size_t groups, size_t stride) {
-            std::vector<double> o(groups);
+        auto compact = [](auto &v, size_t groups, size_t stride) {
+            std::decay_t<decltype(v)> o(groups);
             for (size_t i = 0; i < groups; ++i) o[i] = v[i * stride];
             v.swap(o);
         };
         compact(g.jacob, (size_t)c->K, c->np);
         compact(g.gmetg, (size_t)c->K * 9, c->np);
-        for (int d = 0; d < 3; ++d) compact(g.gmet[d], (size_t)c->K * 3, c->ns);
+        compact(g.gmet, (size_t)c->K * 9, c->ns);
         compact(nhat, (size_t)c->M * 3, c->nf);
         compact(norm, (size_t)c->M, c->nf);
     }
     TRY(upload(c, &c->jacob, g.jacob));
+    if (c->ms) c->h_jacob = std::move(g.jacob);
     TRY(upload(c, &c->gmetg, g.gmetg));
-    for (int d = 0; d < 3; ++d) TRY(upload(c, &c->gmet[d], g.gmet[d]));
+    TRY(upload(c, &c->gmet, g.gmet));
     TRY(upload(c, &c->nhat, nhat));
     TRY(upload(c, &c->norm, norm));
     TRY(upload(c, &c->e2m, e2m));
@@ -3005,11 +2762,11 @@ int dsem_get_metrics(dsem_ctx *c, double *gmetg, double *gmet, double *nhat, dou
                 for (int d = 0; d < 3; ++d)
                     for (size_t s = 0; s < ns; ++s)
                         for (int i = 0; i < 3; ++i)
-                            gmet[((e * 3 + d) * ns + s) * 3 + i] = g.gmet[d][(e * 3 + i) * ns + s];
+                            gmet[((e * 3 + d) * ns + s) * 3 + i] = g.gmet[(e * 9 + d * 3 + i) * ns + s];
         }
     }
     if (nhat || norm) {
-        std::vector<double> nh, nr;
+        dsem::Array nh, nr;
         dsem::mortar_geometry(c->ops, c->M, c->h_corners.data(), c->h_melem.data(), c->h_mface.data(), nh, nr);
         const size_t nf = c->nf;
         for (size_t mm = 0; mm < (size_t)c->M; ++mm)

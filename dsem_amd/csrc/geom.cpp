@@ -151,10 +151,10 @@ bool element_geometry(const Ops &o, int K, const double *corners, Geometry &g)
     const int ncg = o.ncg, nc = o.nc, np = ncg * ncg * ncg, ns = nc * ncg * ncg;
     g.K = K;
     g.p = o.p;
-    g.xg.assign((size_t)K * np * 3, 0.0);
-    g.jacob.assign((size_t)K * np, 0.0);
-    g.gmetg.assign((size_t)K * 9 * np, 0.0);
-    for (int d = 0; d < 3; ++d) g.gmet[d].assign((size_t)K * 3 * ns, 0.0);
+    g.xg.resize((size_t)K * np * 3);
+    g.jacob.resize((size_t)K * np);
+    g.gmetg.resize((size_t)K * 9 * np);
+    g.gmet.resize((size_t)K * 9 * ns);
     bool affine = true;
 #pragma omp parallel for schedule(static) reduction(&& : affine)
     for (int e = 0; e < K; ++e) {
@@ -183,7 +183,7 @@ bool element_geometry(const Ops &o, int K, const double *corners, Geometry &g)
                         else { X[0] = o.cxg[a]; X[1] = o.cxg[b]; X[2] = o.cx[j]; s = a + ncg * (b + ncg * j); }
                         grad_hex8(c, X, gr);
                         const double J = invert(gr, gi);
-                        for (int q = 0; q < 3; ++q) g.gmet[d][((size_t)e * 3 + q) * ns + s] = J * gi[d][q];
+                        for (int q = 0; q < 3; ++q) g.gmet[((size_t)e * 9 + d * 3 + q) * ns + s] = J * gi[d][q];
                     }
         }
     }
@@ -192,12 +192,12 @@ bool element_geometry(const Ops &o, int K, const double *corners, Geometry &g)
 }
 
 void mortar_geometry(const Ops &o, int M, const double *corners, const int32_t *m_elem,
-                     const int32_t *m_face, std::vector<double> &nhat, std::vector<double> &norm)
+                     const int32_t *m_face, Array &nhat, Array &norm)
 {
     static const double end_vals[6] = {0.0, 1.0, 0.0, 1.0, 1.0, 0.0};
     const int ncg = o.ncg, nf = ncg * ncg;
-    nhat.assign((size_t)M * 3 * nf, 0.0);
-    norm.assign((size_t)M * nf, 0.0);
+    nhat.resize((size_t)M * 3 * nf);
+    norm.resize((size_t)M * nf);
 #pragma omp parallel for schedule(static)
     for (int mm = 0; mm < M; ++mm) {
         const int e = m_elem[2 * mm], f = m_face[2 * mm];
