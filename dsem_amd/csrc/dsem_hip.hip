@@ -671,47 +671,6 @@ __device__ __forceinline__ void volume_div(const typename Ctr<PM>::T *sF, const 
     }
 }
 
-// Direct global->LDS copy (global_load_lds_dword): lane l of a wave moves one
-// dword from its own address src to the LDS byte address M0 + 4 l, through no
-// register.  Written as inline asm on purpose: the compiler's own form makes
-// every later LDS read wait for all such copies (it cannot tell the
-// destinations apart), which would serialize the copies with the work they
-// are meant to overlap.  The caller waits for them itself (lds_copies_done)
-// before the barrier that publishes them.  lds_wave_base must be the same for
-// every lane of the wave.
-typedef __attribute__((address_space(3))) void *LdsPtr;
-
-// LDS byte address of an object in shared memory.
-__device__ __forceinline__ unsigned lds_addr(const void *p) { return (unsigned)(size_t)(LdsPtr)p; }
-
-// lds: LDS byte address of the wave's first dword, the same for every lane
-__device__ __forceinline__ void lds_dword(const void *src, unsigned lds)
-{
-    const unsigned l = __builtin_amdgcn_readfirstlane(lds);
-    // The LDS base goes in through the {m0} operand constraint: the compiler
-    // writes M0 itself and knows the copy reads it, so no value of its own is
-    // kept there across the copy.  The s_nop separates that write from the
-    // copy's use of M0.
-    asm volatile("s_nop 0\n\tglobal_load_lds_dword %0, off" : : "v"(src), "{m0}"(l) : "memory");
-}
-
-// The same with a scalar base address (uniform over the wave) and a byte
-// offset per lane.
-__device__ __forceinline__ void lds_dword_s(const void *src, unsigned off, unsigned lds)
-{
-    const unsigned l = __builtin_amdgcn_readfirstlane(lds);
-    asm volatile("s_nop 0\n\tglobal_load_lds_dword %0, %1" : : "v"(off), "s"(src), "{m0}"(l) : "memory");
-}
-
-// s_waitcnt immediate of gfx9 for vmcnt(0) alone (expcnt 7, lgkmcnt 15).
-constexpr int VMCNT0 = 0x0F70;
-
-// Every copy this wave issued has landed in LDS.
-__device__ __forceinline__ void lds_copies_done()
-{
-    asm volatile("s_waitcnt vmcnt(0)" : : : "memory");
-}
-
 // Global loads of one element's state and 1/J and of its six faces'
 // averages, all issued before any use.
 template <int P>
@@ -1665,6 +1624,7 @@ __global__ __launch_bounds__(BLOCK) void k_modal(double *__restrict__ JQ, DevMes
 }
 
 #include "adjoint.inc"
+#include "adjoint_volume.inc"
 
 }  // namespace
 
@@ -1709,7 +1669,7 @@ struct dsem_ctx {
     bool have_lag = false;
     bool keep_lag = false;                     // save the last stage's staggered states without EV
     bool traces_cur = false;                   // T holds the face traces of the current JQ
-    int vol_grid = 0;                          // resident workgroups of the persistent FP64 volume kernel
+    int vol_grid = 0, adj_vol_grid = 0;        // resident workgroups of the persistent FP64 volume kernels
     bool les = false;                          // static Smagorinsky model
     double les_cs = 0.0, les_numax = 0.0;
     double *nut = nullptr, *nut_g = nullptr;   // eddy viscosity on the staggered grids / Gauss points
@@ -2059,12 +2019,13 @@ int modal_dispatch(dsem_ctx *c, int cutoff)
 
 int adjoint_alloc(dsem_ctx *c)
 {
-    if (c->aQVb) return DSEM_OK;
+    if (c->aFTbe) return DSEM_OK;
     const size_t K = c->K, n = K * NEQ * c->np, nfe = K * 6 * NEQ * c->nf;
     const size_t face_blocks = ((size_t)c->M * c->nf + BLOCK - 1) / BLOCK;
-    TRY(dev_alloc(c, &c->aQVb, K * 3 * NEQ * c->ns));
-    TRY(dev_alloc(c, &c->aGVb, K * 3 * 15 * c->ns));
-    TRY(dev_alloc(c, &c->aFTbe, nfe));
+    if (c->p < 5) {   // staggered adjoints between k_adj_volume and k_adj_gather
+        TRY(dev_alloc(c, &c->aQVb, K * 3 * NEQ * c->ns));
+        TRY(dev_alloc(c, &c->aGVb, K * 3 * 15 * c->ns));
+    }
     TRY(dev_alloc(c, &c->aFVb, nfe));
     TRY(dev_alloc(c, &c->aQAbe, nfe));
     TRY(dev_alloc(c, &c->aTb, nfe));
@@ -2075,6 +2036,7 @@ int adjoint_alloc(dsem_ctx *c)
     TRY(dev_alloc(c, &c->aGb, n));
     TRY(dev_alloc(c, &c->aLam, n));
     TRY(dev_alloc(c, &c->aOut, n));
+    TRY(dev_alloc(c, &c->aFTbe, nfe));   // last: marks the set complete
     return DSEM_OK;
 }
 
@@ -2094,6 +2056,24 @@ int adjoint_lag_alloc(dsem_ctx *c)
 struct FwdTape {
     double *T, *QA, *FV;
 };
+
+// Workgroups of the persistent adjoint volume kernel (as volume_grid_size).
+template <int P>
+int adj_volume_grid_size(dsem_ctx *c, int &grid)
+{
+    if constexpr (Vol<P>::MF) {
+        int &g = c->adj_vol_grid;
+        if (g == 0) {
+            int per_cu = 0, ncu = 0;
+            HIP_TRY(c, hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, k_adj_volume_mf<P, 3>, AdjVol<P>::BLK, 0));
+            HIP_TRY(c, hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, c->device));
+            if (per_cu < 1 || ncu < 1) return set_err(c, DSEM_ERR_HIP, "adjoint volume kernel: no resident work-group fits");
+            g = per_cu * ncu;
+        }
+        grid = g < c->K ? g : c->K;
+    }
+    return DSEM_OK;
+}
 
 // Adjoint of one RHS evaluation at state JQ (device) for the cotangent in
 // Gb, with the forward intermediates in f (recomputed first when fwd).
@@ -2122,22 +2102,34 @@ int run_rhs_vjp(dsem_ctx *c, double *JQ, FwdTape f, bool fwd, double *Gb, double
     }
     hipStream_t s = c->stream;
     double *nu_f = c->aNuPart, *nu_v = c->aNuPart + face_blocks;
+    int grid = K;
+    TRY(adj_volume_grid_size<P>(c, grid));
     return launch(c, KID_ADJ, [&] {
         k_adj_update<P><<<K, BLOCK, 0, s>>>(Gb, Qb, cdt, c->aFTbe);
         k_adj_face_visc<P><<<face_blocks, BLOCK, 0, s>>>(c->aFTbe, f.FV, m, ph, c->aFIb, c->aFVb, nu_f);
-        auto vol = [&](auto rot, auto lag) {
-            k_adj_volume<P, (P >= 4), decltype(rot)::value, decltype(lag)::value><<<K, ABLOCK, 0, s>>>(
-                JQ, m, ph, f.QA, muh, Gb, c->aFVb, c->aQVb, c->aGVb, nu_v, MuB, SlagB, nut, NutB);
-        };
-        auto lagged = [&](auto rot) {
-            if (nut) vol(rot, std::integral_constant<int, 2>{});
-            else if (muh || MuB || SlagB) vol(rot, std::integral_constant<int, 1>{});
-            else vol(rot, std::integral_constant<int, 0>{});
-        };
-        if (c->rotated) lagged(std::true_type{});
-        else lagged(std::false_type{});
-        if constexpr (P >= 5) k_adj_gather_dma<P><<<K, GBLOCK, 0, s>>>(m, c->aQVb, c->aGVb, c->aJQvb, c->aQAbe);
-        else k_adj_gather<P><<<K, GBLOCK, 0, s>>>(m, c->aQVb, c->aGVb, c->aJQvb, c->aQAbe);
+        if constexpr (Vol<P>::MF) {
+            auto vol = [&](auto model) {
+                k_adj_volume_mf<P, decltype(model)::value><<<grid, AdjVol<P>::BLK, 0, s>>>(
+                    JQ, m, ph, f.QA, muh, Gb, c->aFVb, c->aJQvb, c->aQAbe, nu_v, MuB, SlagB, nut, NutB);
+            };
+            if (nut && muh) vol(std::integral_constant<int, 3>{});
+            else if (nut) vol(std::integral_constant<int, 2>{});
+            else if (muh) vol(std::integral_constant<int, 1>{});
+            else vol(std::integral_constant<int, 0>{});
+        } else {
+            auto vol = [&](auto rot, auto lag) {
+                k_adj_volume<P, (P >= 4), decltype(rot)::value, decltype(lag)::value><<<K, ABLOCK, 0, s>>>(
+                    JQ, m, ph, f.QA, muh, Gb, c->aFVb, c->aQVb, c->aGVb, nu_v, MuB, SlagB, nut, NutB);
+            };
+            auto lagged = [&](auto rot) {
+                if (nut) vol(rot, std::integral_constant<int, 2>{});
+                else if (muh || MuB || SlagB) vol(rot, std::integral_constant<int, 1>{});
+                else vol(rot, std::integral_constant<int, 0>{});
+            };
+            if (c->rotated) lagged(std::true_type{});
+            else lagged(std::false_type{});
+            k_adj_gather<P><<<K, GBLOCK, 0, s>>>(m, c->aQVb, c->aGVb, c->aJQvb, c->aQAbe);
+        }
         k_adj_face_inv<P><<<face_blocks, BLOCK, 0, s>>>(f.T, m, ph, c->aFIb, c->aQAbe, c->aTb);
         k_adj_traces<P><<<K, BLOCK, 0, s>>>(c->aTb, c->aJQvb, m, Out, Qb, Gb, a, c->aNuPart, face_blocks + K, nu_slot);
     });
@@ -2397,7 +2389,7 @@ void even_odd_ops(const dsem::Ops &o, double *t)
     auto B = [&](int j, int k) { return 0.5 * (o.B[j * n + k] + o.B[(nc - 1 - j) * n + n - 1 - k]); };
     auto D = [&](int k, int j) { return 0.5 * (o.D[k * nc + j] - o.D[(n - 1 - k) * nc + nc - 1 - j]); };
     auto M = [&](int k, int k2) { return 0.5 * (o.M[k * n + k2] - o.M[(n - 1 - k) * n + n - 1 - k2]); };
-    std::fill(t, t + EO_N, 0.0);
+    std::fill(t, t + EO_NADJ, 0.0);
     if constexpr (!Vol<P>::MF) return;
     constexpr int slots = Vol<P>::MIDV ? hg : (n + 1) / 2;   // Gauss pairs that have a slot
     for (int k = 0; k < slots; ++k) {
@@ -2432,6 +2424,36 @@ void even_odd_ops(const dsem::Ops &o, double *t)
         }
         t[EO_GMF] = 0.5 * (D(hg, 0) - D(hg, nc - 1));
     }
+    // transposed operators of the adjoint (rows and slots exchanged)
+    for (int r = 0; r < nrw; ++r) {
+        const int j = j0 + r, jr = nc - 1 - j;
+        const double hj = j == jr ? 0.25 : 0.5;     // a middle row enters as 2 X
+        for (int k = 0; k < slots; ++k) {
+            const int kr = n - 1 - k;
+            const double hk = k == kr ? 0.25 : 0.5;
+            if (j >= 1) {
+                t[EO_TE + r * 4 + k] = -hk * (D(k, j) - D(k, jr));
+                t[EO_TO + r * 4 + k] = k == kr ? 0.0 : -0.5 * (D(k, j) + D(k, jr));
+            }
+            t[EO_XE + k * 4 + r] = hj * (B(j, k) + B(j, kr));
+            t[EO_XO + k * 4 + r] = j == jr ? 0.0 : 0.5 * (B(j, k) - B(j, kr));
+        }
+        if constexpr (Vol<P>::MIDV) t[EO_XM + r] = B(j, hg);
+    }
+    for (int k = 0; k < slots; ++k) {
+        const int kr = n - 1 - k;
+        const double hk = k == kr ? 0.25 : 0.5;
+        if (j0 == 1) {
+            t[EO_XFE + k] = 0.5 * (B(0, k) + B(0, kr));
+            t[EO_XFO + k] = 0.5 * (B(0, k) - B(0, kr));
+        }
+        for (int k2 = 0; k2 < slots; ++k2) {
+            t[EO_HE + k2 * 4 + k] = hk * (M(k, k2) - M(k, n - 1 - k2));
+            t[EO_HO + k2 * 4 + k] = k == kr ? 0.0 : 0.5 * (M(k, k2) + M(k, n - 1 - k2));
+        }
+        t[EO_QF + k] = hk * (D(k, 0) - D(k, nc - 1));
+    }
+    if (Vol<P>::MIDV) t[EO_XFM] = B(0, hg);
     // row sums of the reference operators minus those of the tiles: a
     // constant field c enters the even part as 2 c and the odd part as 0
     auto even_sum = [&](int tile, int row) {
@@ -2494,7 +2516,7 @@ int upload_operators(dsem_ctx *c)
     HIP_TRY(c, hipMemcpyToSymbol(HIP_SYMBOL(c_Bf), Bf, sizeof(Bf)));
     HIP_TRY(c, hipMemcpyToSymbol(HIP_SYMBOL(c_Mf), Mf, sizeof(Mf)));
     HIP_TRY(c, hipMemcpyToSymbol(HIP_SYMBOL(c_Dint), Dint, sizeof(Dint)));
-    double eo[9][EO_N] = {};
+    double eo[9][EO_NADJ] = {};
     {
         dsem::Ops o;
         auto fill = [&](auto p) {
