@@ -58,26 +58,20 @@ def kernel_work(n_elem: int, nmort: int, p: int) -> dict:
     d = 8
     w = {}
     w["k_traces"] = dict(bytes=K * (5 * npt + 6 * 5 * nf) * d, flops=K * 6 * 5 * nf * 2 * ncg)
-    # 192 B per face point: Q_L, Q_R, n, norm in; flux and averaged state out
-    w["k_face_inv"] = dict(bytes=Mm * nf * (10 + 4 + 10) * d, flops=Mm * nf * 120)
     # Bytes: read Q, 1/J and the 9 gradient metrics at Gauss points, the 3
-    # staggered metric rows of each grid, the face averages of the 6 faces
-    # and the face norms; write FV and Qtp.
+    # staggered metric rows of each grid, the face traces (of which each face
+    # also reads its neighbour's) and the face norms; write FV and Qtp.
     w["k_volume"] = dict(bytes=K * (5 * npt + npt + 9 * npt + 3 * 3 * ns + 6 * 5 * nf + 6 * 5 * nf + 5 * npt) * d
                          + Mm * nf * d,
                          flops=K * 180 * nc * ncg ** 3,
                          pointwise_flops=K * 3 * ns * 260)
-    # 128 B per face point: both viscous traces and the norm in, the average out.
-    # The kernel also folds in send_flux_to_faces_add: it reads the Roe flux
-    # and writes FI - average/Re in place of the average (fused: 168 B).
-    w["k_face_visc"] = dict(bytes=Mm * nf * (10 + 1 + 5) * d, flops=Mm * nf * 5 * 6,
-                            fused_bytes=Mm * nf * (10 + 1 + 5 + 5) * d)
-    # 40 B per DOF: Qtp, G, JQ in; G, JQ out.  The fused kernel also reads the
-    # six faces' total fluxes (face part of the divergence) and 1/J, and
-    # writes the next stage's face traces; G is not read by the first stage
+    # 40 B per DOF: Qtp, G, JQ in; G, JQ out.  The fused kernel also reads
+    # both sides' traces and viscous traces (each array counted once), the face
+    # normals and 1/J, forms the face fluxes, and writes the next stage's face
+    # traces; G is not read by the first stage
     # (one launch in five of an RK step).
-    w["k_update"] = dict(bytes=K * npt * 5 * (1 + 2 + 2) * d, flops=K * npt * 5 * 16,
-                         fused_bytes=K * (npt * 5 * (1 + 0.8 + 1 + 2) + npt + 2 * 6 * 5 * nf) * d)
+    w["k_update"] = dict(bytes=K * npt * 5 * (1 + 2 + 2) * d, flops=K * (npt * 5 * 16 + 6 * nf * 150),
+                         fused_bytes=(K * (npt * 5 * (1 + 0.8 + 1 + 2) + npt + 3 * 6 * 5 * nf) + Mm * nf * 4) * d)
     return w
 
 

@@ -1,18 +1,14 @@
 // dsem_hip.hip -- MI355X (gfx950) kernels and C ABI for the DSEM
 // staggered-grid spectral-element RHS and the 5-stage RK4 2N step.
 //
-// Pipeline of one RHS evaluation (one workgroup per element for volume work,
-// one work-item per mortar point for face work; all FP64):
+// Pipeline of one RHS evaluation, one workgroup per element; all FP64:
 //
 //   k_traces        J*Q -> Q, Gauss->Lobatto interpolation evaluated at the
 //                   six faces only (Int_fluxes' face values,
 //                   fluxesH_newa.f90:262-352; send_q_to_mortars, send_q.f90:491-764)
-//   k_face_inv      per mortar point: Roe flux with entropy fix scaled by the
-//                   face norm and the averaged state (interface_flux,
-//                   mortar_operations.f90:151-238; riemann, PhysLib.f90:231-320;
-//                   V_Avg_Soln, mortar_operations.f90:781-837)
 //   k_volume        Gauss-point gradients of Q from the staggered states whose
-//                   face values are the mortar averages (Gauss_Deriv,
+//                   face values are the averages of the two sides' traces
+//                   (V_Avg_Soln, mortar_operations.f90:781-837; Gauss_Deriv,
 //                   SolnDerivsc.f90:14-83, with the combined operator D_int*B
 //                   for the interior Lobatto points), kept in LDS; then per
 //                   staggered grid: interpolated state, prolonged
@@ -22,16 +18,17 @@
 //                   (Int_fluxes fluxesH_newa.f90:274-352, Vis_Fluxes
 //                   Vis_Fluxes_new.f90:84-228, send_flux_to_mortars
 //                   send_flux.f90:243-457, update_interior updatea.f90:100-113)
-//   k_face_visc     per mortar point: averaged viscous flux subtracted from the
-//                   Roe flux (mortar_vis_flux ViscousBC_slide.f90:231-271,
-//                   send_flux_to_faces_add send_flux.f90:699-921)
-//   k_update        face part of the divergence, Qt, and the RK register
-//                   update g = a g + Qt, JQ += c dt g (updatea.f90:213-227)
+//   k_update        face fluxes: Roe flux with entropy fix scaled by the face
+//                   norm (interface_flux, mortar_operations.f90:151-238; riemann,
+//                   PhysLib.f90:231-320) less the averaged viscous flux
+//                   (mortar_vis_flux ViscousBC_slide.f90:231-271,
+//                   send_flux_to_faces_add send_flux.f90:699-921); face part
+//                   of the divergence, Qt, and the RK register update
+//                   g = a g + Qt, JQ += c dt g (updatea.f90:213-227)
 //
 // Element-major structure-of-arrays layouts (ncg = p+1, nc = p+2):
 //   JQ, G, Qtp [K][5][np]        point n + ncg*(m + ncg*l)
 //   T, FV      [K][6][5][nf]     face traces, face f-1, point i + ncg*j
-//   QA, FI, FT [M][5][nf]        per mortar (master face indexing)
 //   metrics    jacob [K][npm], gmetg [K][9][npm], gmet [K][3 grids][3][nsm],
 //              nhat [M][3][nfm], norm [M][nfm]; npm = np (per point) or 1
 //              (per element, affine meshes) -- selected by the stride ms.
@@ -127,6 +124,8 @@ struct DevMesh {
     int rot;                      // some mortar face is rotated (orientation != 0)
     const double *jacob, *gmetg, *gmet;
     const int *e2m;               // [K][6] (mortar << 4) | (map << 1) | side, see e2m_mortar
+    const int *e2n;               // [K][6] neighbour (element face index << 3) | map, see e2n_off
+    const int *eflag;             // [K][6] EF_* bits
     const int *m_elem, *m_face, *m_sign, *m_nsign;
     const int *m_orient;          // [M] slave orientation 0..7, or null when every mortar is aligned
     const double *nhat, *norm;
@@ -189,6 +188,21 @@ __device__ __forceinline__ int orient_point(int o, int q)
 __device__ __forceinline__ int e2m_mortar(int c) { return c >> 4; }
 __device__ __forceinline__ int e2m_map(int c) { return (c >> 1) & 7; }
 
+// Offset in a face array [K][6][5][nf] of what the neighbour across a face
+// holds at the element's own face value vq = v nf + q (n: the face's e2n entry).
+template <int P>
+__device__ __forceinline__ size_t e2n_off(int n, int rot, int vq)
+{
+    constexpr int NF = Sz<P>::NF;
+    const int o = rot ? (vq / NF) * NF + orient_point<Sz<P>::NCG>(n & 7, vq % NF) : vq;
+    return (size_t)(n >> 3) * (NEQ * NF) + o;
+}
+
+// An element face's part in its mortar: it is the slave; its state is the left
+// one of the Roe flux; the slave's viscous trace changes sign; the mortar flux
+// changes sign on this face.
+enum { EF_SLAVE = 1, EF_LEFT = 2, EF_FLIP = 4, EF_NEG = 8 };
+
 // ------------------------------------------------------------ pointwise physics
 // Pointwise physics.  Euler fluxes: fflux/gflux/hflux (PhysLib.f90:17-124).
 // Viscous fluxes x/y/z_vis_flux (PhysLib.f90:419-583), split so that the
@@ -247,9 +261,12 @@ __device__ __forceinline__ void roe_flux(const DevPhys &ph, double n0, double n1
     const double gamma = ph.gamma;
     const double rho = Ql[0], rhon = Qr[0];
     const double ul = Ql[1] / rho, vl = Ql[2] / rho, wl = Ql[3] / rho;
-    const double pleft = (gamma - 1.0) * (Ql[4] - 0.5 / rho * (Ql[1] * Ql[1] + Ql[2] * Ql[2] + Ql[3] * Ql[3]));
+    double pleft = (gamma - 1.0) * (Ql[4] - 0.5 / rho * (Ql[1] * Ql[1] + Ql[2] * Ql[2] + Ql[3] * Ql[3]));
     const double ur = Qr[1] / rhon, vr = Qr[2] / rhon, wr = Qr[3] / rhon;
-    const double pright = (gamma - 1.0) * (Qr[4] - 0.5 / rhon * (Qr[1] * Qr[1] + Qr[2] * Qr[2] + Qr[3] * Qr[3]));
+    double pright = (gamma - 1.0) * (Qr[4] - 0.5 / rhon * (Qr[1] * Qr[1] + Qr[2] * Qr[2] + Qr[3] * Qr[3]));
+    // both rounded before their difference: with one product inside a fused
+    // difference, equal pressures would differ by its rounding
+    asm("" : "+v"(pleft), "+v"(pright));
     const double ql = n0 * ul + n1 * vl + n2 * wl;
     const double qr = n0 * ur + n1 * vr + n2 * wr;
     const double gg = gamma / (gamma - 1.0);
@@ -337,37 +354,6 @@ __global__ __launch_bounds__(BLOCK) void k_traces(const double *__restrict__ JQ,
     }
 }
 
-template <int P>
-__global__ __launch_bounds__(BLOCK) void k_face_inv(const double *__restrict__ T, DevMesh m, DevPhys ph,
-                                                     double *__restrict__ FI, double *__restrict__ QA)
-{
-    using S = Sz<P>;
-    const int idx = blockIdx.x * BLOCK + threadIdx.x;
-    if (idx >= m.M * S::NF) return;
-    const int mm = idx / S::NF, q = idx % S::NF;
-    const int em = m.m_elem[2 * mm], es = m.m_elem[2 * mm + 1];
-    const int fm = m.m_face[2 * mm], fs = m.m_face[2 * mm + 1];
-    double Qm[5], Qs[5], fl[5];
-    const int qs = m.m_orient ? orient_point<S::NCG>(m.m_orient[mm], q) : q;   // rotate_to_mortar
-#pragma unroll
-    for (int v = 0; v < 5; ++v) {
-        Qm[v] = T[(((size_t)em * 6 + fm - 1) * NEQ + v) * S::NF + q];
-        Qs[v] = T[(((size_t)es * 6 + fs - 1) * NEQ + v) * S::NF + qs];
-    }
-    const int nfm = m.ms ? S::NF : 1, qq = q * m.ms;
-    const double n0 = m.nhat[((size_t)mm * 3 + 0) * nfm + qq];
-    const double n1 = m.nhat[((size_t)mm * 3 + 1) * nfm + qq];
-    const double n2 = m.nhat[((size_t)mm * 3 + 2) * nfm + qq];
-    const double ds = m.norm[(size_t)mm * nfm + qq];
-    if (fm == 1 || fm == 3 || fm == 6) roe_flux(ph, n0, n1, n2, ds, Qs, Qm, fl);
-    else roe_flux(ph, n0, n1, n2, ds, Qm, Qs, fl);
-#pragma unroll
-    for (int v = 0; v < 5; ++v) {
-        FI[((size_t)mm * NEQ + v) * S::NF + q] = fl[v];
-        QA[((size_t)mm * NEQ + v) * S::NF + q] = (Qm[v] + Qs[v]) * 0.5;
-    }
-}
-
 // Line contractions of the adjoint volume kernel on the matrix cores.
 // v_mfma_f64_4x4x4f64 runs four independent 4x4x4 products per wave.  Lane l
 // (c = l%4, blk = (l/4)%4, r = l/16) supplies A_blk[c][r] and B_blk[r][c]
@@ -452,9 +438,9 @@ __device__ __forceinline__ double mf_line(const double *fld, const MfLane<P, ROW
 // nc*ncg^2 points of grid D into LDS (interior) or the viscous face traces
 // (faces).
 template <int P, int D, int PM>
-__device__ __forceinline__ void volume_grid(const DevMesh &m, const DevPhys &ph, const double *__restrict__ QA,
+__device__ __forceinline__ void volume_grid(const DevMesh &m, const DevPhys &ph,
                                             const double *__restrict__ muh, const double *__restrict__ nut,
-                                            double *__restrict__ FV, double *__restrict__ Slag,
+                                            double *FV, double *__restrict__ Slag,
                                             const typename Ctr<PM>::T *sQ,
                                             const typename Ctr<PM>::T *sG, typename Ctr<PM>::T *sF,
                                             const double *sBar, const typename Ctr<PM>::T *sB, int e,
@@ -515,7 +501,7 @@ __device__ __forceinline__ void volume_grid(const DevMesh &m, const DevPhys &ph,
 #pragma unroll
         for (int i = 0; i < 3; ++i) vg[i] = gmd[i * nsm + s * m.ms];
 #pragma unroll
-        for (int v = 0; v < 5; ++v) vqa[v] = QA[((size_t)mo * NEQ + v) * S::NF + qm];
+        for (int v = 0; v < 5; ++v) vqa[v] = FV[(((size_t)e * 6 + fc - 1) * NEQ + v) * S::NF + q];
         vnrm = m.norm[(size_t)mo * nfm + qm * m.ms];
         double Qv[5];
         CT Bj[S::NCG];
@@ -671,48 +657,7 @@ __device__ __forceinline__ void volume_div(const typename Ctr<PM>::T *sF, const 
     }
 }
 
-// Global loads of one element's state and 1/J and of its six faces'
-// averages, all issued before any use.
-template <int P>
-__device__ __forceinline__ void volume_inputs(const double *__restrict__ JQ, const double *__restrict__ QA,
-                                              const DevMesh &m, int e, int tid,
-                                              double (&qv)[(NEQ * Sz<P>::NP + VBLOCK - 1) / VBLOCK],
-                                              double (&jv)[(NEQ * Sz<P>::NP + VBLOCK - 1) / VBLOCK],
-                                              double (&av)[(6 * NEQ * Sz<P>::NF + VBLOCK - 1) / VBLOCK])
-{
-    using S = Sz<P>;
-    constexpr int NQV = NEQ * S::NP, NAV = 6 * NEQ * S::NF;
-    constexpr int NQI = (NQV + VBLOCK - 1) / VBLOCK, NAI = (NAV + VBLOCK - 1) / VBLOCK;
-    const double *q = JQ + (size_t)e * NEQ * S::NP;
-    const double *jac = m.jacob + (size_t)e * (m.ms ? S::NP : 1);
-    const int *e2m = m.e2m + (size_t)e * 6;
-    int mort[6], map6[6];
-#pragma unroll
-    for (int f = 0; f < 6; ++f) {
-        mort[f] = e2m_mortar(e2m[f]);
-        map6[f] = e2m_map(e2m[f]);
-    }
-#pragma unroll
-    for (int u = 0; u < NQI; ++u) {
-        const int i = tid + u * VBLOCK;
-        qv[u] = i < NQV ? q[i] : 0.0;
-        jv[u] = i < NQV ? jac[(i % S::NP) * m.ms] : 0.0;
-    }
-#pragma unroll
-    for (int u = 0; u < NAI; ++u) {
-        const int i = tid + u * VBLOCK;
-        const int f = i / (NEQ * S::NF), vq = i % (NEQ * S::NF);
-        // mortar of face f+1 by selects (a dynamic index into mort[] would go to scratch)
-        int mo = mort[0], mp = map6[0];
-#pragma unroll
-        for (int g = 1; g < 6; ++g) {
-            mo = f == g ? mort[g] : mo;
-            mp = f == g ? map6[g] : mp;
-        }
-        const int vqm = m.rot ? (vq / S::NF) * S::NF + orient_point<S::NCG>(mp, vq % S::NF) : vq;
-        av[u] = i < NAV ? QA[(size_t)mo * NEQ * S::NF + vqm] : 0.0;
-    }
-}
+#include "volume.inc"
 
 // Mixed-precision volume kernel (PM 1, 2): Gauss-point gradients into LDS
 // (Gauss_Deriv, SolnDerivsc.f90:14-83), then for each staggered grid the
@@ -730,8 +675,8 @@ __device__ __forceinline__ void volume_inputs(const double *__restrict__ JQ, con
 // Pointwise physics, the RK state and all face kernels stay FP64.
 template <int P, int PM>
 __global__ __launch_bounds__(VBLOCK, 4) void k_volume(const double *__restrict__ JQ, DevMesh m, DevPhys ph,
-                                                      const double *__restrict__ QA, const double *__restrict__ muh,
-                                                      const double *__restrict__ nut, double *__restrict__ FV,
+                                                      const double *__restrict__ T, const double *__restrict__ muh,
+                                                      const double *__restrict__ nut, double *FV,
                                                       double *__restrict__ Qtp, double *__restrict__ Slag)
 {
     using S = Sz<P>;
@@ -750,8 +695,7 @@ __global__ __launch_bounds__(VBLOCK, 4) void k_volume(const double *__restrict__
     __shared__ CT sOp[NOP];
     __shared__ double sDint[S::NCG];          // sum over interior j of D[k][j]
     const int tid = threadIdx.x, e = blockIdx.x;
-    constexpr int NQV = NEQ * S::NP, NAV = 6 * NEQ * S::NF;
-    constexpr int NQI = (NQV + VBLOCK - 1) / VBLOCK, NAI = (NAV + VBLOCK - 1) / VBLOCK;
+    constexpr int NFV = NEQ * S::NF, NAV = 6 * NFV;
     constexpr int NOI = (NOP + VBLOCK - 1) / VBLOCK;
 #pragma unroll
     for (int u = 0; u < NOI; ++u) {
@@ -767,8 +711,13 @@ __global__ __launch_bounds__(VBLOCK, 4) void k_volume(const double *__restrict__
     // ---- prologue.  Every global load of the element's inputs is issued
     // before the first wait: one exposed memory latency per element instead
     // of one per loop trip.
-    double qv[NQI], jv[NQI], av[NAI];
-    volume_inputs<P>(JQ, QA, m, e, tid, qv, jv, av);
+    const int *e2n = m.e2n + (size_t)e * 6;
+    const int nb0 = e2n[0], nb1 = e2n[1], nb2 = e2n[2], nb3 = e2n[3], nb4 = e2n[4], nb5 = e2n[5];
+    VolInputs<P, VBLOCK> in;
+    in.load(JQ, T, m.jacob, m.ms, m.rot, e, [=](int f) {
+        // by selects: an array with a dynamic index would go to scratch
+        return f < 3 ? (f == 0 ? nb0 : (f == 1 ? nb1 : nb2)) : (f == 3 ? nb3 : (f == 4 ? nb4 : nb5));
+    }, tid);
     {
         // metric rows of this work-item's Gauss points, first used after the
         // gradient contractions: unconditional loads from a clamped point,
@@ -813,14 +762,21 @@ __global__ __launch_bounds__(VBLOCK, 4) void k_volume(const double *__restrict__
     }
     CT *sQA = sF;   // face averages of the six faces minus Qbar (face f+1 at [f][v][q])
 #pragma unroll
-    for (int u = 0; u < NQI; ++u) {
-        const int i = tid + u * VBLOCK;
-        if (i < NQV) sQ[i] = (CT)(qv[u] * jv[u] - sBar[i / S::NP]);
+    for (int r = 0; r < R; ++r) {
+        const int pt = tid + r * VBLOCK;
+        if (pt < S::NP)
+#pragma unroll
+            for (int v = 0; v < 5; ++v) sQ[v * S::NP + pt] = (CT)(in.q[r][v] * in.j[r] - sBar[v]);
     }
 #pragma unroll
-    for (int u = 0; u < NAI; ++u) {
+    for (int u = 0; u < in.NAI; ++u) {
         const int i = tid + u * VBLOCK;
-        if (i < NAV) sQA[i] = (CT)(av[u] - sBar[(i % (NEQ * S::NF)) / S::NF]);
+        if (i < NAV) {
+            const double a = in.face(u);
+            sQA[i] = (CT)(a - sBar[(i % NFV) / S::NF]);
+            // the FP64 averages wait where the face points' traces will go
+            FV[(size_t)e * NAV + i] = a;
+        }
     }
     __syncthreads();
 
@@ -867,11 +823,11 @@ __global__ __launch_bounds__(VBLOCK, 4) void k_volume(const double *__restrict__
     for (int r = 0; r < R; ++r)
 #pragma unroll
         for (int v = 0; v < 5; ++v) acc[r][v] = 0.0;
-    volume_grid<P, 0, PM>(m, ph, QA, muh, nut, FV, Slag, sQ, sG, sF, sBar, sOp + OB, e, e2m_e, tid);
+    volume_grid<P, 0, PM>(m, ph, muh, nut, FV, Slag, sQ, sG, sF, sBar, sOp + OB, e, e2m_e, tid);
     volume_div<P, 0, PM>(sF, sOp + OD, sBar, sDint, tid, acc);
-    volume_grid<P, 1, PM>(m, ph, QA, muh, nut, FV, Slag, sQ, sG, sF, sBar, sOp + OB, e, e2m_e, tid);
+    volume_grid<P, 1, PM>(m, ph, muh, nut, FV, Slag, sQ, sG, sF, sBar, sOp + OB, e, e2m_e, tid);
     volume_div<P, 1, PM>(sF, sOp + OD, sBar, sDint, tid, acc);
-    volume_grid<P, 2, PM>(m, ph, QA, muh, nut, FV, Slag, sQ, sG, sF, sBar, sOp + OB, e, e2m_e, tid);
+    volume_grid<P, 2, PM>(m, ph, muh, nut, FV, Slag, sQ, sG, sF, sBar, sOp + OB, e, e2m_e, tid);
     volume_div<P, 2, PM>(sF, sOp + OD, sBar, sDint, tid, acc);
 #pragma unroll
     for (int r = 0; r < R; ++r) {
@@ -882,31 +838,6 @@ __global__ __launch_bounds__(VBLOCK, 4) void k_volume(const double *__restrict__
     }
 }
 
-#include "volume.inc"
-
-template <int P>
-__global__ __launch_bounds__(BLOCK) void k_face_visc(const double *__restrict__ FV, const double *__restrict__ FI,
-                                                      DevMesh m, DevPhys ph, double *__restrict__ FT)
-{
-    using S = Sz<P>;
-    const int idx = blockIdx.x * BLOCK + threadIdx.x;
-    if (idx >= m.M * S::NF) return;
-    const int mm = idx / S::NF, q = idx % S::NF;
-    const int em = m.m_elem[2 * mm], es = m.m_elem[2 * mm + 1];
-    const int fm = m.m_face[2 * mm], fs = m.m_face[2 * mm + 1];
-    const int nfm = m.ms ? S::NF : 1;
-    const double nrm = m.norm[(size_t)mm * nfm + q * m.ms];
-    const bool flip = m.m_nsign[mm] == -1;
-    const int qs = m.m_orient ? orient_point<S::NCG>(m.m_orient[mm], q) : q;   // rotate_fv_to_mortar
-#pragma unroll
-    for (int v = 0; v < 5; ++v) {
-        const double fvm = FV[(((size_t)em * 6 + fm - 1) * NEQ + v) * S::NF + q];
-        double fvs = FV[(((size_t)es * 6 + fs - 1) * NEQ + v) * S::NF + qs];
-        if (flip) fvs = -fvs;
-        const double qb = 0.5 * (fvm + fvs) * nrm;
-        FT[((size_t)mm * NEQ + v) * S::NF + q] = FI[((size_t)mm * NEQ + v) * S::NF + q] - qb / ph.re;
-    }
-}
 
 struct StageArgs {
     double a, cdt;                 // RK coefficients for this stage (a unused when first)
@@ -916,34 +847,52 @@ struct StageArgs {
     unsigned int *nonfinite;       // set when any Qt is NaN/Inf (nullable)
 };
 
-// Face part of the divergence, Qt, and (rk) the register update
-// g = a g + Qt, JQ += c dt g (updatea.f90:213-227).  With TRACES the updated
-// state is staged in LDS and the face traces of the next stage are computed
-// here, so the state is not read again by k_traces.
-// HBM-bound: 512 work-items per element and UBLK independent points per
-// work-item in flight (all loads of a batch issued before any store), so that
-// enough bytes are outstanding per CU to approach the HBM bandwidth.
-constexpr int UBLOCK = 512;
-constexpr int UBLK = 4;
+// Face fluxes, the face part of the divergence, Qt, and (rk) the register update
+// g = a g + Qt, JQ += c dt g (updatea.f90:213-227).  Both elements of a mortar
+// form its flux, from the traces T (Roe flux with entropy fix) and the viscous
+// traces FV of both sides in the master's order, so the two results are the
+// same to the last bit.  With TRACES the updated state is staged in LDS and the
+// face traces of the next stage are computed here, into the other trace array
+// (neighbours may still read T), so the state is not read again by k_traces.
+//
+// HBM-bound.  A face kernel before and after the volume kernel moved the same
+// bytes (averages, Roe and total fluxes per mortar, written and read) in two
+// more launches: 22^3 p = 8 367 + 117 + 75 us per evaluation against 475 here,
+// 1320 elements p = 7 33.5 + 10.1 + 8.2 against 45.4, 4199 p = 3 20.0 + 9.0 +
+// 6.9 against 29.3, 8^3 p = 6 12.4 + 5.7 + 4.9 against 15.0; 16^3 p = 6
+// 66 + 24 + 20 against 115, with two launches less.
+// Work-items: what the element's points keep busy with two loads in flight
+// each, so that enough workgroups share a CU (p = 3: 512 work-items 41 us, 128 to
+// 192 30 us).  The face points' 25 loads come first and are used up before the
+// batches start: with the first batch in flight behind the Roe flux the
+// registers spill (22^3 p = 8 535 us).
+template <int P>
+struct Upd {
+    static constexpr int BLK = P >= 5 ? 512 : P == 4 ? 384 : P == 3 ? 192 : P == 2 ? 128 : 64;
+    static constexpr int UB = 2;    // points of a batch, all loads of which are issued before a store
+    static constexpr int WPE = 4;   // waves per SIMD the registers must allow
+};
 
-// One batch of UBLK points of k_update: Qtp, and for an RK stage G, JQ and
+// One batch of points of k_update: Qtp, and for an RK stage G, JQ and
 // (with traces) 1/J.  Indices past the element are clamped in range; the
 // caller skips those points.
+template <int P>
 struct UpdBatch {
-    double q[UBLK], g[UBLK], j[UBLK], c[UBLK];
+    static constexpr int UB = Upd<P>::UB;
+    double q[UB], g[UB], j[UB], c[UB];
 };
 
 template <int P, bool TRACES>
-__device__ __forceinline__ UpdBatch upd_load(const double *__restrict__ Qtp, const double *__restrict__ G,
+__device__ __forceinline__ UpdBatch<P> upd_load(const double *__restrict__ Qtp, const double *__restrict__ G,
                                              const double *__restrict__ JQ, const double *__restrict__ jac, int ms,
                                              const StageArgs &st, size_t e0, int base)
 {
     using S = Sz<P>;
     constexpr int NQ = NEQ * S::NP;
-    UpdBatch bt;
+    UpdBatch<P> bt;
 #pragma unroll
-    for (int u = 0; u < UBLK; ++u) {
-        const int i = base + u * UBLOCK;
+    for (int u = 0; u < Upd<P>::UB; ++u) {
+        const int i = base + u * Upd<P>::BLK;
         const int ic = i < NQ ? i : NQ - 1;
         bt.q[u] = Qtp[e0 + ic];
         bt.g[u] = (st.rk && !st.first) ? G[e0 + ic] : 0.0;
@@ -954,75 +903,79 @@ __device__ __forceinline__ UpdBatch upd_load(const double *__restrict__ Qtp, con
 }
 
 template <int P, bool TRACES>
-__global__ __launch_bounds__(UBLOCK) void k_update(const double *__restrict__ Qtp, const double *__restrict__ FT, DevMesh m,
-                                                    StageArgs st, double *__restrict__ JQ, double *__restrict__ G,
-                                                    double *__restrict__ Qt, double *__restrict__ T)
+__global__ __launch_bounds__((Upd<P>::BLK), (Upd<P>::WPE)) void k_update(const double *__restrict__ Qtp, const double *__restrict__ T,
+                                                    const double *__restrict__ FV, DevMesh m, DevPhys ph, StageArgs st,
+                                                    double *__restrict__ JQ, double *__restrict__ G,
+                                                    double *__restrict__ Qt, double *__restrict__ Tnext)
 {
     using S = Sz<P>;
-    constexpr int NQ = NEQ * S::NP, NFT = 6 * NEQ * S::NF;
-    constexpr int NFI = (NFT + UBLOCK - 1) / UBLOCK;            // face values per work-item
-    constexpr int NTRIP = (NQ + UBLOCK * UBLK - 1) / (UBLOCK * UBLK);
+    constexpr int NQ = NEQ * S::NP, NFV = NEQ * S::NF, NFT = 6 * NFV;
+    constexpr int BLK = Upd<P>::BLK, NTRIP = (NQ + BLK * Upd<P>::UB - 1) / (BLK * Upd<P>::UB);
+    static_assert(6 * S::NF <= BLK, "one face point per work-item");
     __shared__ double sFT[NFT];
     __shared__ double sQ[TRACES ? NQ : 1];
     __shared__ double sDf[2 * S::NCG];   // D[k][0], D[k][nc-1]: face part of the divergence
     __shared__ double sBf[2 * S::NCG];   // B[0][k], B[nc-1][k]: face traces
     const int e = blockIdx.x, tid = threadIdx.x;
-    // Mortar and orientation sign of the six faces: uniform per element, so
-    // these are scalar loads; each work-item picks its face by selects.
-    const int *e2m = m.e2m + (size_t)e * 6;
-    int fmo[6], fmp[6];
-    double fsg[6];
+    // Tables of the six faces: uniform per element, so these are scalar loads;
+    // each work-item picks its face by selects.
+    const int f = tid / S::NF, q = tid % S::NF;
+    const bool isf = f < 6;
+    int c = m.e2m[(size_t)e * 6], nb = m.e2n[(size_t)e * 6], fl = m.eflag[(size_t)e * 6];
 #pragma unroll
-    for (int f = 0; f < 6; ++f) {
-        const int c = e2m[f];
-        fmo[f] = e2m_mortar(c);
-        fmp[f] = e2m_map(c);
-        fsg[f] = ((c & 1) && m.m_sign[e2m_mortar(c)] == -1) ? -1.0 : 1.0;
+    for (int g = 1; g < 6; ++g) {
+        c = f == g ? m.e2m[(size_t)e * 6 + g] : c;
+        nb = f == g ? m.e2n[(size_t)e * 6 + g] : nb;
+        fl = f == g ? m.eflag[(size_t)e * 6 + g] : fl;
     }
-    // Every global load of the face fluxes and of the first batch of points
-    // is issued before the first wait.
-    double fv[NFI];
+    double Ql[5], Qr[5], fo[5], fn[5], n0 = 0.0, n1 = 0.0, n2 = 0.0, ds = 0.0;
+    if (isf) {
+        const size_t own = (size_t)e * NFT + f * NFV + q, nbr = e2n_off<P>(nb, m.rot, q);
+        const size_t ol = (fl & EF_LEFT) ? own : nbr, orr = (fl & EF_LEFT) ? nbr : own;
 #pragma unroll
-    for (int u = 0; u < NFI; ++u) {
-        const int i = tid + u * UBLOCK;
-        const int f = i / (NEQ * S::NF), r = i % (NEQ * S::NF);
-        int mo = fmo[0], mp = fmp[0];
-#pragma unroll
-        for (int g = 1; g < 6; ++g) {
-            mo = f == g ? fmo[g] : mo;
-            mp = f == g ? fmp[g] : mp;
+        for (int v = 0; v < 5; ++v) {
+            Ql[v] = T[ol + v * S::NF];
+            Qr[v] = T[orr + v * S::NF];
+            fo[v] = FV[own + v * S::NF];
+            fn[v] = FV[nbr + v * S::NF];
         }
-        const int rm = m.rot ? (r / S::NF) * S::NF + orient_point<S::NCG>(mp, r % S::NF) : r;   // rotate_flux_to_face
-        fv[u] = i < NFT ? FT[(size_t)mo * NEQ * S::NF + rm] : 0.0;
+        const int nfm = m.ms ? S::NF : 1, qq = (m.rot ? orient_point<S::NCG>(e2m_map(c), q) : q) * m.ms;
+        const size_t mo = e2m_mortar(c);
+        n0 = m.nhat[(mo * 3 + 0) * nfm + qq];
+        n1 = m.nhat[(mo * 3 + 1) * nfm + qq];
+        n2 = m.nhat[(mo * 3 + 2) * nfm + qq];
+        ds = m.norm[mo * nfm + qq];
     }
     const double *jac = m.jacob + (size_t)e * (m.ms ? S::NP : 1);
     const size_t e0 = (size_t)e * NQ;
-    UpdBatch bt = upd_load<P, TRACES>(Qtp, G, JQ, jac, m.ms, st, e0, tid);
     if (tid < S::NCG) {
         sDf[tid] = c_D[P][tid * S::NC];
         sDf[S::NCG + tid] = c_D[P][tid * S::NC + S::NC - 1];
         sBf[tid] = c_B[P][tid];
         sBf[S::NCG + tid] = c_B[P][(S::NC - 1) * S::NCG + tid];
     }
+    if (isf) {
+        double fx[5];
+        roe_flux(ph, n0, n1, n2, ds, Ql, Qr, fx);
+        const bool fo_neg = (fl & EF_FLIP) && (fl & EF_SLAVE), fn_neg = (fl & EF_FLIP) && !(fl & EF_SLAVE);
 #pragma unroll
-    for (int u = 0; u < NFI; ++u) {
-        const int i = tid + u * UBLOCK;
-        const int f = i / (NEQ * S::NF);
-        double sg = fsg[0];
-#pragma unroll
-        for (int g = 1; g < 6; ++g) sg = f == g ? fsg[g] : sg;
-        if (i < NFT) sFT[i] = sg < 0.0 ? -fv[u] : fv[u];
+        for (int v = 0; v < 5; ++v) {
+            const double qb = 0.5 * ((fo_neg ? -fo[v] : fo[v]) + (fn_neg ? -fn[v] : fn[v])) * ds;
+            asm("" : "+v"(fx[v]));   // rounded before the difference, as the reference stores it
+            const double t = fx[v] - qb / ph.re;
+            sFT[f * NFV + v * S::NF + q] = (fl & EF_NEG) ? -t : t;
+        }
     }
     __syncthreads();
     double mx = 0.0;
     bool bad = false;
 #pragma unroll
     for (int trip = 0; trip < NTRIP; ++trip) {
-        const int base = tid + trip * UBLOCK * UBLK;
-        if (trip > 0) bt = upd_load<P, TRACES>(Qtp, G, JQ, jac, m.ms, st, e0, base);
+        const int base = tid + trip * BLK * Upd<P>::UB;
+        const UpdBatch<P> bt = upd_load<P, TRACES>(Qtp, G, JQ, jac, m.ms, st, e0, base);
 #pragma unroll
-        for (int u = 0; u < UBLK; ++u) {
-            const int i = base + u * UBLOCK;
+        for (int u = 0; u < Upd<P>::UB; ++u) {
+            const int i = base + u * Upd<P>::BLK;
             if (i >= NQ) continue;
             const int v = i / S::NP, pt = i % S::NP;
             const int n = pt % S::NCG, mi = (pt / S::NCG) % S::NCG, l = pt / (S::NCG * S::NCG);
@@ -1054,8 +1007,8 @@ __global__ __launch_bounds__(UBLOCK) void k_update(const double *__restrict__ Qt
     if (st.resid && e == m.K - 1) atomicMax(st.resid, (unsigned long long)__double_as_longlong(mx));
     if (TRACES) {
         __syncthreads();
-        double *t = T + (size_t)e * NFT;
-        for (int i = tid; i < NFT; i += UBLOCK) {
+        double *t = Tnext + (size_t)e * NFT;
+        for (int i = tid; i < NFT; i += BLK) {
             const int qf = i % S::NF, v = (i / S::NF) % NEQ, f = i / (NEQ * S::NF) + 1;
             const int a = qf % S::NCG, b = qf / S::NCG;
             const int d = (f == 4 || f == 6) ? 0 : ((f == 1 || f == 2) ? 1 : 2);
@@ -1636,6 +1589,8 @@ namespace {
 const double kArk[5] = {0.0, -0.4178904745, -1.192151694643, -1.697784692471, -1.514183444257};
 const double kCrk[5] = {0.1496590219993, 0.3792103129999, 0.8229550293869, 0.6994504559488, 0.1530572479681};
 
+// The table of names is part of the interface: the face kernels keep their
+// entries, with no launches, since k_update forms the face fluxes.
 enum KernelId { KID_TRACES = 0, KID_FACE_INV, KID_VOLUME, KID_FACE_VISC, KID_UPDATE, KID_DTCALC, KID_EV, KID_DIAG, KID_ADJ, KID_LES, KID_MODAL, KID_COUNT };
 const char *const kKernelNames[KID_COUNT] = {"k_traces", "k_face_inv", "k_volume", "k_face_visc",
                                              "k_update", "k_dtcalc", "k_ev", "k_diag", "k_adj", "k_smag",
@@ -1662,7 +1617,7 @@ struct dsem_ctx {
     std::vector<int32_t> h_melem, h_mface;
     // device buffers
     double *JQ = nullptr, *G = nullptr, *Qtp = nullptr, *Qt = nullptr;
-    double *T = nullptr, *FV = nullptr, *QA = nullptr, *FI = nullptr, *FT = nullptr;
+    double *T = nullptr, *Tnext = nullptr, *FV = nullptr;   // k_update reads T of its neighbours and writes Tnext
     double *jacob = nullptr, *gmetg = nullptr, *gmet = nullptr;
     double *nhat = nullptr, *norm = nullptr, *muh = nullptr;
     double *Slag = nullptr, *muhg = nullptr, *ev_resid = nullptr, *ev_ducros = nullptr;   // entropy viscosity
@@ -1689,10 +1644,10 @@ struct dsem_ctx {
     std::vector<int> tape_sens;                // per tape slot: the Smagorinsky sensor switches
     bool tape_les = false;                     // the tape's slots hold nu_t (the layout of tape_reserve)
     // step tape: per slot and stage the stage input state and the forward
-    // intermediates the adjoint reads (face traces T, mortar averages QA,
-    // viscous face traces FV)
+    // intermediates the adjoint reads (face traces T, viscous face traces FV)
     double *tape = nullptr;
     int tape_slots = 0;
+    int *e2n = nullptr, *eflag = nullptr;
     int *e2m = nullptr, *m_elem = nullptr, *m_face = nullptr, *m_sign = nullptr, *m_nsign = nullptr;
     int *m_orient = nullptr;                   // [M] orientation codes, allocated only when some face is rotated
     bool rotated = false;                      // some mortar has orientation != 0
@@ -1746,7 +1701,7 @@ DevMesh dev_mesh(const dsem_ctx *c)
     DevMesh m;
     m.K = c->K; m.M = c->M; m.ms = c->ms;
     m.jacob = c->jacob; m.gmetg = c->gmetg; m.gmet = c->gmet;
-    m.e2m = c->e2m; m.m_elem = c->m_elem; m.m_face = c->m_face; m.m_sign = c->m_sign; m.m_nsign = c->m_nsign;
+    m.e2m = c->e2m; m.e2n = c->e2n; m.eflag = c->eflag; m.m_elem = c->m_elem; m.m_face = c->m_face; m.m_sign = c->m_sign; m.m_nsign = c->m_nsign;
     m.m_orient = c->m_orient;
     m.rot = c->rotated ? 1 : 0;
     m.nhat = c->nhat; m.norm = c->norm;
@@ -1820,10 +1775,10 @@ int volume_grid_size(dsem_ctx *c, int &grid)
 // and the partial residual Qtp.  Every entry a call reads is written earlier
 // in the same call, so none needs clearing.
 struct RhsBufs {
-    double *T, *QA, *FI, *FV, *FT, *Qtp;
+    double *T, *Tnext, *FV, *Qtp;
 };
 
-RhsBufs ctx_bufs(const dsem_ctx *c) { return RhsBufs{c->T, c->QA, c->FI, c->FV, c->FT, c->Qtp}; }
+RhsBufs ctx_bufs(const dsem_ctx *c) { return RhsBufs{c->T, c->Tnext, c->FV, c->Qtp}; }
 
 // The instance of the FP64 volume kernel for this call's viscosities.
 template <int P>
@@ -1834,9 +1789,9 @@ void run_volume64(dsem_ctx *c, const double *JQ, const DevMesh &m, const DevPhys
         constexpr int MODEL = decltype(model)::value;
         constexpr bool LAG = decltype(lag)::value;
         if constexpr (Vol<P>::MF)
-            k_volume_mf<P, MODEL, LAG><<<grid, Vol<P>::BLK, 0, c->stream>>>(JQ, m, ph, b.QA, muh, nut, b.FV, b.Qtp, slag);
+            k_volume_mf<P, MODEL, LAG><<<grid, Vol<P>::BLK, 0, c->stream>>>(JQ, m, ph, b.T, muh, nut, b.FV, b.Qtp, slag);
         else
-            k_volume_vec<P, MODEL, LAG><<<grid, Vol<P>::BLK, 0, c->stream>>>(JQ, m, ph, b.QA, muh, nut, b.FV, b.Qtp, slag);
+            k_volume_vec<P, MODEL, LAG><<<grid, Vol<P>::BLK, 0, c->stream>>>(JQ, m, ph, b.T, muh, nut, b.FV, b.Qtp, slag);
     };
     auto lagged = [&](auto model) {
         if (slag) go(model, std::true_type{});
@@ -1861,29 +1816,32 @@ int run_rhs(dsem_ctx *c, double *JQ, const StageArgs &st, double *Qt_out, bool t
     const DevMesh m = dev_mesh(c);
     const DevPhys ph = dev_phys(c);
     const int K = c->K;
-    const int face_blocks = (c->M * S::NF + BLOCK - 1) / BLOCK;
     const double *muh = c->params.shock ? c->muh : nullptr;
     const double *nut = c->les ? c->nut : nullptr;
     hipStream_t s = c->stream;
     c->traces_cur = false;   // only dsem_rk_steps vouches for T after its last stage
     if (!traces_ready) TRY(launch(c, KID_TRACES, [&] { k_traces<P><<<K, BLOCK, 0, s>>>(JQ, m, b.T); }));
-    TRY(launch(c, KID_FACE_INV, [&] { k_face_inv<P><<<face_blocks, BLOCK, 0, s>>>(b.T, m, ph, b.FI, b.QA); }));
     double *slag = save_lag ? c->Slag : nullptr;
     int grid = K;
     if (c->params.precision == DSEM_PREC_FP64) TRY(volume_grid_size<P>(c, grid));
     TRY(launch(c, KID_VOLUME, [&] {
         if (c->params.precision == DSEM_PREC_FP32)
-            k_volume<P, 1><<<K, VBLOCK, 0, s>>>(JQ, m, ph, b.QA, muh, nut, b.FV, b.Qtp, slag);
+            k_volume<P, 1><<<K, VBLOCK, 0, s>>>(JQ, m, ph, b.T, muh, nut, b.FV, b.Qtp, slag);
         else if (c->params.precision == DSEM_PREC_BF16X3)
-            k_volume<P, 2><<<K, VBLOCK, 0, s>>>(JQ, m, ph, b.QA, muh, nut, b.FV, b.Qtp, slag);
+            k_volume<P, 2><<<K, VBLOCK, 0, s>>>(JQ, m, ph, b.T, muh, nut, b.FV, b.Qtp, slag);
         else
             run_volume64<P>(c, JQ, m, ph, b, muh, nut, slag, grid);
     }));
-    TRY(launch(c, KID_FACE_VISC, [&] { k_face_visc<P><<<face_blocks, BLOCK, 0, s>>>(b.FV, b.FI, m, ph, b.FT); }));
-    if (make_traces)
-        TRY(launch(c, KID_UPDATE, [&] { k_update<P, true><<<K, UBLOCK, 0, s>>>(b.Qtp, b.FT, m, st, JQ, c->G, Qt_out, b.T); }));
-    else
-        TRY(launch(c, KID_UPDATE, [&] { k_update<P, false><<<K, UBLOCK, 0, s>>>(b.Qtp, b.FT, m, st, JQ, c->G, Qt_out, b.T); }));
+    if (make_traces) {
+        TRY(launch(c, KID_UPDATE, [&] {
+            k_update<P, true><<<K, Upd<P>::BLK, 0, s>>>(b.Qtp, b.T, b.FV, m, ph, st, JQ, c->G, Qt_out, b.Tnext);
+        }));
+        std::swap(c->T, c->Tnext);
+    } else {
+        TRY(launch(c, KID_UPDATE, [&] {
+            k_update<P, false><<<K, Upd<P>::BLK, 0, s>>>(b.Qtp, b.T, b.FV, m, ph, st, JQ, c->G, Qt_out, nullptr);
+        }));
+    }
     return DSEM_OK;
 }
 
@@ -2054,7 +2012,7 @@ int adjoint_lag_alloc(dsem_ctx *c)
 
 // Forward intermediates of one RHS evaluation that its adjoint reads.
 struct FwdTape {
-    double *T, *QA, *FV;
+    double *T, *FV;
 };
 
 // Workgroups of the persistent adjoint volume kernel (as volume_grid_size).
@@ -2097,8 +2055,8 @@ int run_rhs_vjp(dsem_ctx *c, double *JQ, FwdTape f, bool fwd, double *Gb, double
     const int face_blocks = (c->M * S::NF + BLOCK - 1) / BLOCK;
     if (fwd) {
         StageArgs st{0.0, 0.0, 0, 0, nullptr, nullptr};
-        TRY(run_rhs<P>(c, JQ, st, c->Qt, false, false, false, ctx_bufs(c)));   // forward intermediates in c->T, QA, FV
-        f = FwdTape{c->T, c->QA, c->FV};
+        TRY(run_rhs<P>(c, JQ, st, c->Qt, false, false, false, ctx_bufs(c)));   // forward intermediates in c->T, FV
+        f = FwdTape{c->T, c->FV};
     }
     hipStream_t s = c->stream;
     double *nu_f = c->aNuPart, *nu_v = c->aNuPart + face_blocks;
@@ -2110,7 +2068,7 @@ int run_rhs_vjp(dsem_ctx *c, double *JQ, FwdTape f, bool fwd, double *Gb, double
         if constexpr (Vol<P>::MF) {
             auto vol = [&](auto model) {
                 k_adj_volume_mf<P, decltype(model)::value><<<grid, AdjVol<P>::BLK, 0, s>>>(
-                    JQ, m, ph, f.QA, muh, Gb, c->aFVb, c->aJQvb, c->aQAbe, nu_v, MuB, SlagB, nut, NutB);
+                    JQ, m, ph, f.T, muh, Gb, c->aFVb, c->aJQvb, c->aQAbe, nu_v, MuB, SlagB, nut, NutB);
             };
             if (nut && muh) vol(std::integral_constant<int, 3>{});
             else if (nut) vol(std::integral_constant<int, 2>{});
@@ -2119,7 +2077,7 @@ int run_rhs_vjp(dsem_ctx *c, double *JQ, FwdTape f, bool fwd, double *Gb, double
         } else {
             auto vol = [&](auto rot, auto lag) {
                 k_adj_volume<P, (P >= 4), decltype(rot)::value, decltype(lag)::value><<<K, ABLOCK, 0, s>>>(
-                    JQ, m, ph, f.QA, muh, Gb, c->aFVb, c->aQVb, c->aGVb, nu_v, MuB, SlagB, nut, NutB);
+                    JQ, m, ph, f.T, muh, Gb, c->aFVb, c->aQVb, c->aGVb, nu_v, MuB, SlagB, nut, NutB);
             };
             auto lagged = [&](auto rot) {
                 if (nut) vol(rot, std::integral_constant<int, 2>{});
@@ -2199,12 +2157,11 @@ int les_vjp_dispatch(dsem_ctx *c, const double *JQ, const double *Slag, double c
     DISPATCH_P(c, run_les_vjp, JQ, Slag, cs, numax, sensors, NutB, JQb, SlagB, nu_slot);
 }
 
-// Tape layout per slot and stage: state [n], T [nT], QA [nQA], FV [nT].
+// Tape layout per slot and stage: state [n], T [nT], FV [nT].
 size_t tape_stage_size(const dsem_ctx *c)
 {
     const size_t n = (size_t)c->K * NEQ * c->np, nT = (size_t)c->K * 6 * NEQ * c->nf;
-    const size_t nQA = (size_t)c->M * NEQ * c->nf;
-    return n + 2 * nT + nQA;
+    return n + 2 * nT;
 }
 
 // After a slot's five stages: with entropy viscosity the step's mu_h
@@ -2236,12 +2193,10 @@ void tape_ev(const dsem_ctx *c, int slot, double **muh, double **slag, double **
 void tape_stage(const dsem_ctx *c, int slot, int k, double **S, FwdTape *f)
 {
     const size_t n = (size_t)c->K * NEQ * c->np, nT = (size_t)c->K * 6 * NEQ * c->nf;
-    const size_t nQA = (size_t)c->M * NEQ * c->nf;
     double *b = c->tape + (size_t)slot * tape_slot_size(c) + (size_t)k * tape_stage_size(c);
     *S = b;
     f->T = b + n;
-    f->QA = b + n + nT;
-    f->FV = b + n + nT + nQA;
+    f->FV = b + n + nT;
 }
 
 int tape_reserve(dsem_ctx *c, int nslots)
@@ -2272,7 +2227,7 @@ int tape_reserve(dsem_ctx *c, int nslots)
 int record_step(dsem_ctx *c, double dt, int slot)
 {
     const size_t n = (size_t)c->K * NEQ * c->np;
-    double *T0 = c->T, *QA0 = c->QA, *FV0 = c->FV;
+    double *T0 = c->T, *FV0 = c->FV;
     int rc = DSEM_OK;
     if (c->les != c->tape_les)
         return set_err(c, DSEM_ERR_ARG, "the Smagorinsky switch changed since dsem_tape_reserve: reserve again");
@@ -2316,12 +2271,10 @@ int record_step(dsem_ctx *c, double dt, int slot)
         st.resid = nullptr;
         st.nonfinite = nullptr;
         c->T = f.T;
-        c->QA = f.QA;
         c->FV = f.FV;
         // the last stage leaves the next step's lagged states, as dsem_rk_steps does
         rc = rhs_dispatch(c, c->JQ, st, nullptr, false, false, (lag_model || c->keep_lag) && k == 4);
         c->T = T0;
-        c->QA = QA0;
         c->FV = FV0;
     }
     if (rc == DSEM_OK && (lag_model || c->keep_lag)) c->have_lag = true;
@@ -2608,6 +2561,18 @@ int create_impl(const dsem_mesh_desc *mesh, const dsem_params *prm, int device, 
     for (size_t i = 0; i < e2m.size(); ++i)
         if (e2m[i] < 0) return set_err(c, DSEM_ERR_UNSUPPORTED, "open element face: boundary conditions are not part of this path");
 
+    std::vector<int> e2n(e2m.size()), eflag(e2m.size());
+    for (int k = 0; k < c->M; ++k) {
+        const int *el = &me[2 * (size_t)k], *fa = &mf[2 * (size_t)k];
+        const bool swap = fa[0] == 1 || fa[0] == 3 || fa[0] == 6;   // the slave's state is the left one
+        for (int s = 0; s < 2; ++s) {
+            const size_t own = (size_t)el[s] * 6 + fa[s] - 1, nbr = (size_t)el[1 - s] * 6 + fa[1 - s] - 1;
+            e2n[own] = (int)(nbr << 3) | (s == 0 ? mor[k] : ((e2m[own] >> 1) & 7));
+            eflag[own] = (s ? EF_SLAVE : 0) | ((s == 0) != swap ? EF_LEFT : 0) | (mns[k] == -1 ? EF_FLIP : 0) |
+                         (s && msg[k] == -1 ? EF_NEG : 0);
+        }
+    }
+
     HIP_TRY(c, hipSetDevice(device));
     HIP_TRY(c, hipStreamCreate(&c->stream));
     TRY(scratch_setup(c));
@@ -2650,6 +2615,8 @@ int create_impl(const dsem_mesh_desc *mesh, const dsem_params *prm, int device, 
     TRY(upload(c, &c->nhat, nhat));
     TRY(upload(c, &c->norm, norm));
     TRY(upload(c, &c->e2m, e2m));
+    TRY(upload(c, &c->e2n, e2n));
+    TRY(upload(c, &c->eflag, eflag));
     TRY(upload(c, &c->m_elem, me));
     TRY(upload(c, &c->m_face, mf));
     TRY(upload(c, &c->m_sign, msg));
@@ -2662,9 +2629,7 @@ int create_impl(const dsem_mesh_desc *mesh, const dsem_params *prm, int device, 
     TRY(dev_alloc(c, &c->Qt, nst));
     TRY(dev_alloc(c, &c->T, (size_t)c->K * 6 * NEQ * c->nf));
     TRY(dev_alloc(c, &c->FV, (size_t)c->K * 6 * NEQ * c->nf));
-    TRY(dev_alloc(c, &c->QA, (size_t)c->M * NEQ * c->nf));
-    TRY(dev_alloc(c, &c->FI, (size_t)c->M * NEQ * c->nf));
-    TRY(dev_alloc(c, &c->FT, (size_t)c->M * NEQ * c->nf));
+    TRY(dev_alloc(c, &c->Tnext, (size_t)c->K * 6 * NEQ * c->nf));
     TRY(dev_alloc(c, &c->muh, (size_t)c->K * 3 * c->ns));
     TRY(dev_alloc(c, &c->muhg, (size_t)c->K * c->np));
     TRY(upload(c, &c->bmat, dsem::ke_weights(c->ops)));
@@ -3012,8 +2977,9 @@ int dsem_rhs_device_noalloc(dsem_ctx *c, const double *dJQ, double *dQt)
 {
     if (!c || !c->stream || !dJQ || !dQt) return set_err(c, DSEM_ERR_ARG, "rhs_device_noalloc arguments");
     if (!c->scratch) return set_err(c, DSEM_ERR_ARG, "no scratch address for this device");
-    // T, FV [K][6][5][nf]; QA, FI, FT [M][5][nf]; Qtp [K][5][np]; each part
-    // starts on a 256-byte boundary
+    // T, FV [K][6][5][nf]; Qtp [K][5][np]; each part starts on a 256-byte
+    // boundary.  The declared need, which callers size their meshes by, counts
+    // three mortar arrays more.
     size_t used = 0;
     auto take = [&](size_t n) {
         double *p = c->scratch + used;
@@ -3023,11 +2989,10 @@ int dsem_rhs_device_noalloc(dsem_ctx *c, const double *dJQ, double *dQt)
     const size_t nface = (size_t)c->K * 6 * NEQ * c->nf, nmort = (size_t)c->M * NEQ * c->nf;
     RhsBufs b;
     b.T = take(nface);
+    b.Tnext = nullptr;   // no traces of a next state on this path
     b.FV = take(nface);
-    b.QA = take(nmort);
-    b.FI = take(nmort);
-    b.FT = take(nmort);
     b.Qtp = take((size_t)c->K * NEQ * c->np);
+    for (int i = 0; i < 3; ++i) (void)take(nmort);
     if (used * sizeof(double) > DSEM_NOALLOC_SCRATCH_BYTES)
         return set_err(c, DSEM_ERR_ARG, "rhs_device_noalloc: this mesh needs " + std::to_string(used * sizeof(double)) +
                                             " bytes of scratch, more than the " +
@@ -3121,7 +3086,7 @@ int dsem_rhs_vjp_device(dsem_ctx *c, const double *dJQ, const double *dLam, doub
 {
     TRY(vjp_check(c));
     if (!dJQ || !dLam || !dJQbar) return set_err(c, DSEM_ERR_ARG, "rhs_vjp_device pointers");
-    TRY(rhs_vjp_dispatch(c, const_cast<double *>(dJQ), FwdTape{nullptr, nullptr, nullptr}, true,
+    TRY(rhs_vjp_dispatch(c, const_cast<double *>(dJQ), FwdTape{nullptr, nullptr}, true,
                          const_cast<double *>(dLam), nullptr, 0.0, 0.0, dJQbar, c->aNu));
     double h = 0.0;
     HIP_TRY(c, hipMemcpyAsync(&h, c->aNu, sizeof(double), hipMemcpyDeviceToHost, c->stream));
