@@ -842,17 +842,17 @@ __global__ __launch_bounds__(VBLOCK, 4) void k_volume(const double *__restrict__
 struct StageArgs {
     double a, cdt;                 // RK coefficients for this stage (a unused when first)
     int first;                     // first stage: g = Qt
-    int rk;                        // 0: write Qt only, 1: RK update
     unsigned long long *resid;     // max |Qt| of the last element (nullable)
     unsigned int *nonfinite;       // set when any Qt is NaN/Inf (nullable)
 };
 
-// Face fluxes, the face part of the divergence, Qt, and (rk) the register update
-// g = a g + Qt, JQ += c dt g (updatea.f90:213-227).  Both elements of a mortar
+// Face fluxes, the face part of the divergence, and Qt (MODE 0) or the register
+// update g = a g + Qt, JQ += c dt g (updatea.f90:213-227), in place in JQnext
+// (MODE 1) or from JQ to JQnext (MODE 2, a recorded step's next tape state).  Both elements of a mortar
 // form its flux, from the traces T (Roe flux with entropy fix) and the viscous
 // traces FV of both sides in the master's order, so the two results are the
-// same to the last bit.  With TRACES the updated state is staged in LDS and the
-// face traces of the next stage are computed here, into the other trace array
+// same to the last bit.  The updated state is staged in LDS and the face traces
+// of the next stage are computed here, into the other trace array
 // (neighbours may still read T), so the state is not read again by k_traces.
 //
 // HBM-bound.  A face kernel before and after the volume kernel moved the same
@@ -882,7 +882,7 @@ struct UpdBatch {
     double q[UB], g[UB], j[UB], c[UB];
 };
 
-template <int P, bool TRACES>
+template <int P, bool RK>
 __device__ __forceinline__ UpdBatch<P> upd_load(const double *__restrict__ Qtp, const double *__restrict__ G,
                                              const double *__restrict__ JQ, const double *__restrict__ jac, int ms,
                                              const StageArgs &st, size_t e0, int base)
@@ -895,25 +895,27 @@ __device__ __forceinline__ UpdBatch<P> upd_load(const double *__restrict__ Qtp, 
         const int i = base + u * Upd<P>::BLK;
         const int ic = i < NQ ? i : NQ - 1;
         bt.q[u] = Qtp[e0 + ic];
-        bt.g[u] = (st.rk && !st.first) ? G[e0 + ic] : 0.0;
-        bt.j[u] = st.rk ? JQ[e0 + ic] : 0.0;
-        bt.c[u] = (st.rk && TRACES) ? jac[(ic % S::NP) * ms] : 0.0;
+        bt.g[u] = (RK && !st.first) ? G[e0 + ic] : 0.0;
+        bt.j[u] = RK ? JQ[e0 + ic] : 0.0;
+        bt.c[u] = RK ? jac[(ic % S::NP) * ms] : 0.0;
     }
     return bt;
 }
 
-template <int P, bool TRACES>
+template <int P, int MODE>
 __global__ __launch_bounds__((Upd<P>::BLK), (Upd<P>::WPE)) void k_update(const double *__restrict__ Qtp, const double *__restrict__ T,
                                                     const double *__restrict__ FV, DevMesh m, DevPhys ph, StageArgs st,
-                                                    double *__restrict__ JQ, double *__restrict__ G,
+                                                    const double *__restrict__ JQ, double *__restrict__ JQnext,
+                                                    double *__restrict__ G,
                                                     double *__restrict__ Qt, double *__restrict__ Tnext)
 {
     using S = Sz<P>;
+    constexpr bool RK = MODE != 0;
     constexpr int NQ = NEQ * S::NP, NFV = NEQ * S::NF, NFT = 6 * NFV;
     constexpr int BLK = Upd<P>::BLK, NTRIP = (NQ + BLK * Upd<P>::UB - 1) / (BLK * Upd<P>::UB);
     static_assert(6 * S::NF <= BLK, "one face point per work-item");
     __shared__ double sFT[NFT];
-    __shared__ double sQ[TRACES ? NQ : 1];
+    __shared__ double sQ[RK ? NQ : 1];
     __shared__ double sDf[2 * S::NCG];   // D[k][0], D[k][nc-1]: face part of the divergence
     __shared__ double sBf[2 * S::NCG];   // B[0][k], B[nc-1][k]: face traces
     const int e = blockIdx.x, tid = threadIdx.x;
@@ -972,7 +974,7 @@ __global__ __launch_bounds__((Upd<P>::BLK), (Upd<P>::WPE)) void k_update(const d
 #pragma unroll
     for (int trip = 0; trip < NTRIP; ++trip) {
         const int base = tid + trip * BLK * Upd<P>::UB;
-        const UpdBatch<P> bt = upd_load<P, TRACES>(Qtp, G, JQ, jac, m.ms, st, e0, base);
+        const UpdBatch<P> bt = upd_load<P, RK>(Qtp, G, MODE == 1 ? JQnext : JQ, jac, m.ms, st, e0, base);
 #pragma unroll
         for (int u = 0; u < Upd<P>::UB; ++u) {
             const int i = base + u * Upd<P>::BLK;
@@ -990,12 +992,14 @@ __global__ __launch_bounds__((Upd<P>::BLK), (Upd<P>::WPE)) void k_update(const d
                 const double F1 = sFT[((face_of<P>(d, 1) - 1) * NEQ + v) * S::NF + q];
                 qt = qt - fma(sDf[k], F0, sDf[S::NCG + k] * F1);
             }
-            if (st.rk) {
+            // JQnext is set in every RK mode: the branch keeps the compiler from
+            // gathering the batch's stores (480 us without it, 470 with)
+            if (RK && JQnext) {
                 const double g = st.first ? qt : fma(st.a, bt.g[u], qt);
                 G[e0 + i] = g;
                 const double jq = fma(st.cdt, g, bt.j[u]);
-                JQ[e0 + i] = jq;
-                if (TRACES) sQ[i] = jq * bt.c[u];
+                JQnext[e0 + i] = jq;
+                sQ[i] = jq * bt.c[u];
             } else {
                 Qt[e0 + i] = qt;
             }
@@ -1005,7 +1009,7 @@ __global__ __launch_bounds__((Upd<P>::BLK), (Upd<P>::WPE)) void k_update(const d
     }
     if (bad && st.nonfinite) atomicOr(st.nonfinite, 1u);
     if (st.resid && e == m.K - 1) atomicMax(st.resid, (unsigned long long)__double_as_longlong(mx));
-    if (TRACES) {
+    if constexpr (RK) {
         __syncthreads();
         double *t = Tnext + (size_t)e * NFT;
         for (int i = tid; i < NFT; i += BLK) {
@@ -1624,6 +1628,7 @@ struct dsem_ctx {
     bool have_lag = false;
     bool keep_lag = false;                     // save the last stage's staggered states without EV
     bool traces_cur = false;                   // T holds the face traces of the current JQ
+    bool state_lent = false;                   // dsem_state_pointers gave JQ out: a caller may write it
     int vol_grid = 0, adj_vol_grid = 0;        // resident workgroups of the persistent FP64 volume kernels
     bool les = false;                          // static Smagorinsky model
     double les_cs = 0.0, les_numax = 0.0;
@@ -1776,6 +1781,7 @@ int volume_grid_size(dsem_ctx *c, int &grid)
 // in the same call, so none needs clearing.
 struct RhsBufs {
     double *T, *Tnext, *FV, *Qtp;
+    double *JQnext = nullptr;   // where an RK stage leaves the state, null: in place
 };
 
 RhsBufs ctx_bufs(const dsem_ctx *c) { return RhsBufs{c->T, c->Tnext, c->FV, c->Qtp}; }
@@ -1804,12 +1810,11 @@ void run_volume64(dsem_ctx *c, const double *JQ, const DevMesh &m, const DevPhys
 }
 
 // One RHS evaluation on state JQ; the final kernel either writes Qt or
-// performs an RK register update (st.rk).
-// traces_ready: T already holds the face traces of JQ (computed by the
-// previous stage's update); make_traces: this stage's update also computes
-// the traces of the updated state for the next stage.
+// performs an RK register update (rk), which also leaves the traces of the
+// updated state in b.Tnext.  traces_ready: b.T already holds the face traces of
+// JQ (left by the previous stage's update).
 template <int P>
-int run_rhs(dsem_ctx *c, double *JQ, const StageArgs &st, double *Qt_out, bool traces_ready, bool make_traces,
+int run_rhs(dsem_ctx *c, double *JQ, const StageArgs &st, double *Qt_out, bool traces_ready, bool rk,
             bool save_lag, const RhsBufs &b)
 {
     using S = Sz<P>;
@@ -1819,7 +1824,7 @@ int run_rhs(dsem_ctx *c, double *JQ, const StageArgs &st, double *Qt_out, bool t
     const double *muh = c->params.shock ? c->muh : nullptr;
     const double *nut = c->les ? c->nut : nullptr;
     hipStream_t s = c->stream;
-    c->traces_cur = false;   // only dsem_rk_steps vouches for T after its last stage
+    c->traces_cur = false;   // the callers vouch for T after an RK step's last stage
     if (!traces_ready) TRY(launch(c, KID_TRACES, [&] { k_traces<P><<<K, BLOCK, 0, s>>>(JQ, m, b.T); }));
     double *slag = save_lag ? c->Slag : nullptr;
     int grid = K;
@@ -1832,17 +1837,14 @@ int run_rhs(dsem_ctx *c, double *JQ, const StageArgs &st, double *Qt_out, bool t
         else
             run_volume64<P>(c, JQ, m, ph, b, muh, nut, slag, grid);
     }));
-    if (make_traces) {
-        TRY(launch(c, KID_UPDATE, [&] {
-            k_update<P, true><<<K, Upd<P>::BLK, 0, s>>>(b.Qtp, b.T, b.FV, m, ph, st, JQ, c->G, Qt_out, b.Tnext);
-        }));
-        std::swap(c->T, c->Tnext);
-    } else {
-        TRY(launch(c, KID_UPDATE, [&] {
-            k_update<P, false><<<K, Upd<P>::BLK, 0, s>>>(b.Qtp, b.T, b.FV, m, ph, st, JQ, c->G, Qt_out, nullptr);
-        }));
-    }
-    return DSEM_OK;
+    return launch(c, KID_UPDATE, [&] {
+        auto go = [&](auto mode, const double *src, double *dst, double *Tn) {
+            k_update<P, decltype(mode)::value><<<K, Upd<P>::BLK, 0, s>>>(b.Qtp, b.T, b.FV, m, ph, st, src, dst, c->G, Qt_out, Tn);
+        };
+        if (!rk) go(std::integral_constant<int, 0>{}, nullptr, nullptr, nullptr);
+        else if (!b.JQnext) go(std::integral_constant<int, 1>{}, nullptr, JQ, b.Tnext);
+        else go(std::integral_constant<int, 2>{}, JQ, b.JQnext, b.Tnext);
+    });
 }
 
 template <int P>
@@ -1867,10 +1869,10 @@ int run_dtcalc(dsem_ctx *c, unsigned long long *out)
     }
 
 int rhs_dispatch(dsem_ctx *c, double *JQ, const StageArgs &st, double *Qt_out, bool traces_ready = false,
-                 bool make_traces = false, bool save_lag = false, const RhsBufs *bufs = nullptr)
+                 bool rk = false, bool save_lag = false, const RhsBufs *bufs = nullptr)
 {
     const RhsBufs b = bufs ? *bufs : ctx_bufs(c);
-    DISPATCH_P(c, run_rhs, JQ, st, Qt_out, traces_ready, make_traces, save_lag, b);
+    DISPATCH_P(c, run_rhs, JQ, st, Qt_out, traces_ready, rk, save_lag, b);
 }
 
 template <int P>
@@ -2054,7 +2056,7 @@ int run_rhs_vjp(dsem_ctx *c, double *JQ, FwdTape f, bool fwd, double *Gb, double
     const int K = c->K;
     const int face_blocks = (c->M * S::NF + BLOCK - 1) / BLOCK;
     if (fwd) {
-        StageArgs st{0.0, 0.0, 0, 0, nullptr, nullptr};
+        StageArgs st{0.0, 0.0, 0, nullptr, nullptr};
         TRY(run_rhs<P>(c, JQ, st, c->Qt, false, false, false, ctx_bufs(c)));   // forward intermediates in c->T, FV
         f = FwdTape{c->T, c->FV};
     }
@@ -2227,8 +2229,8 @@ int tape_reserve(dsem_ctx *c, int nslots)
 int record_step(dsem_ctx *c, double dt, int slot)
 {
     const size_t n = (size_t)c->K * NEQ * c->np;
-    double *T0 = c->T, *FV0 = c->FV;
     int rc = DSEM_OK;
+    const bool ready = c->traces_cur && !c->state_lent;   // c->T holds the traces of c->JQ
     if (c->les != c->tape_les)
         return set_err(c, DSEM_ERR_ARG, "the Smagorinsky switch changed since dsem_tape_reserve: reserve again");
     const bool lag_model = c->params.shock || c->les;
@@ -2261,24 +2263,32 @@ int record_step(dsem_ctx *c, double dt, int slot)
         double *S;
         FwdTape f;
         tape_stage(c, slot, k, &S, &f);
-        hipError_t e = hipMemcpyAsync(S, c->JQ, sizeof(double) * n, hipMemcpyDeviceToDevice, c->stream);
-        if (e != hipSuccess) { rc = set_err(c, DSEM_ERR_HIP, hipGetErrorString(e)); break; }
+        if (k == 0) {
+            HIP_TRY(c, hipMemcpyAsync(S, c->JQ, sizeof(double) * n, hipMemcpyDeviceToDevice, c->stream));
+            if (ready)
+                HIP_TRY(c, hipMemcpyAsync(f.T, c->T, sizeof(double) * (size_t)c->K * 6 * NEQ * c->nf,
+                                          hipMemcpyDeviceToDevice, c->stream));
+        }
         StageArgs st;
         st.a = kArk[k];
         st.cdt = kCrk[k] * dt;
         st.first = (k == 0);
-        st.rk = 1;
         st.resid = nullptr;
         st.nonfinite = nullptr;
-        c->T = f.T;
-        c->FV = f.FV;
+        // each stage leaves its state and traces where the next one is recorded,
+        // the last one in the context
+        RhsBufs b = ctx_bufs(c);
+        FwdTape fn{c->T, nullptr};
+        b.JQnext = c->JQ;
+        if (k < 4) tape_stage(c, slot, k + 1, &b.JQnext, &fn);
+        b.T = f.T;
+        b.Tnext = fn.T;
+        b.FV = f.FV;
         // the last stage leaves the next step's lagged states, as dsem_rk_steps does
-        rc = rhs_dispatch(c, c->JQ, st, nullptr, false, false, (lag_model || c->keep_lag) && k == 4);
-        c->T = T0;
-        c->FV = FV0;
+        rc = rhs_dispatch(c, S, st, nullptr, k > 0 || ready, true, (lag_model || c->keep_lag) && k == 4, &b);
     }
     if (rc == DSEM_OK && (lag_model || c->keep_lag)) c->have_lag = true;
-    c->traces_cur = false;
+    c->traces_cur = rc == DSEM_OK && !c->state_lent;
     return rc;
 }
 
@@ -2969,7 +2979,7 @@ int dsem_rhs_device(dsem_ctx *c, const double *dJQ, double *dQt)
 {
     if (!c || !c->stream || !dJQ || !dQt) return set_err(c, DSEM_ERR_ARG, "rhs_device arguments");
     HIP_TRY(c, hipSetDevice(c->device));
-    StageArgs st{0.0, 0.0, 0, 0, nullptr, nullptr};
+    StageArgs st{0.0, 0.0, 0, nullptr, nullptr};
     return rhs_dispatch(c, const_cast<double *>(dJQ), st, dQt);
 }
 
@@ -2999,7 +3009,7 @@ int dsem_rhs_device_noalloc(dsem_ctx *c, const double *dJQ, double *dQt)
                                             std::to_string((unsigned long long)DSEM_NOALLOC_SCRATCH_BYTES) +
                                             " bytes of the static array (use dsem_rhs_device)");
     HIP_TRY(c, hipSetDevice(c->device));
-    StageArgs st{0.0, 0.0, 0, 0, nullptr, nullptr};
+    StageArgs st{0.0, 0.0, 0, nullptr, nullptr};
     return rhs_dispatch(c, const_cast<double *>(dJQ), st, dQt, false, false, false, &b);
 }
 
@@ -3008,7 +3018,7 @@ int dsem_rhs(dsem_ctx *c, double t, double *Qt_out)
     (void)t;   // no time-dependent source terms on this path (source terms = none)
     if (!c || !c->stream) return set_err(c, DSEM_ERR_ARG, "rhs arguments");
     HIP_TRY(c, hipSetDevice(c->device));
-    StageArgs st{0.0, 0.0, 0, 0, nullptr, nullptr};
+    StageArgs st{0.0, 0.0, 0, nullptr, nullptr};
     TRY(rhs_dispatch(c, c->JQ, st, c->Qt));
     if (Qt_out) {
         HIP_TRY(c, hipMemcpyAsync(Qt_out, c->Qt, sizeof(double) * (size_t)c->K * NEQ * c->np, hipMemcpyDeviceToHost,
@@ -3033,7 +3043,6 @@ int dsem_rk_steps(dsem_ctx *c, double t, double dt, int nsteps, double *resid_ou
             st.a = kArk[k];
             st.cdt = kCrk[k] * dt;
             st.first = (k == 0);
-            st.rk = 1;
             const bool last = check && s == nsteps - 1 && k == 4;
             st.resid = last ? &c->d_scalars[0] : nullptr;
             st.nonfinite = check ? reinterpret_cast<unsigned int *>(&c->d_scalars[2]) : nullptr;
@@ -3043,6 +3052,7 @@ int dsem_rk_steps(dsem_ctx *c, double t, double dt, int nsteps, double *resid_ou
             // updated state for the next stage or call.
             const bool ready = (s == 0 && k == 0) ? c->traces_cur : true;
             TRY(rhs_dispatch(c, c->JQ, st, nullptr, ready, true, (c->params.shock || c->keep_lag || c->les) && k == 4));
+            std::swap(c->T, c->Tnext);
         }
         if (c->params.shock || c->keep_lag || c->les) c->have_lag = true;
     }
@@ -3271,7 +3281,10 @@ int dsem_dtcalc(dsem_ctx *c, double *dt_out)
 int dsem_state_pointers(dsem_ctx *c, double **dJQ, double **dG)
 {
     if (!c) return DSEM_ERR_ARG;
-    if (dJQ) *dJQ = c->JQ;
+    if (dJQ) {
+        *dJQ = c->JQ;
+        c->state_lent = true;
+    }
     if (dG) *dG = c->G;
     return DSEM_OK;
 }

@@ -38,3 +38,34 @@ def test_rotated_faces_rhs_and_steps(p, metrics, tol):
     e1, e2 = rel_l2(rhs, O.rhs(g, JQ, ph)), rel_l2(got - JQ, ref - JQ)
     print("rhs", e1, "steps", e2, flush=True)
     assert np.all(e1 <= tol) and np.all(e2 <= tol)
+
+
+@pytest.mark.parametrize("p", range(1, 9))
+def test_recorded_steps_are_the_plain_steps(p):
+    """A recorded step leaves each stage's state and traces in the tape and the
+    last ones in the context: the state after recorded and plain steps in turn,
+    and after a write to the state in between, equals plain steps bit for bit."""
+    print(f"\n[case] recorded steps p={p}", flush=True)
+    mesh = M.rotated_box(3, p, seed=p)
+    with DSEM(mesh, re=400.0) as s:
+        xg, jac = s.gauss_points()
+        JQ = cases.tgv_state(xg, jac, "isothermal", perturb=1e-2, seed=p)
+        s.set_state(JQ)
+        dt = 0.3 * s.dtcalc()
+        s.steps(4, dt)
+        want = s.get_state()
+        s.tape_reserve(2)
+        for recorded in ((True, True, False, True), (False, True, False, False)):
+            s.set_state(JQ)
+            for i, rec in enumerate(recorded):
+                if rec:
+                    s.rk_step_record(dt, i % 2)
+                else:
+                    s.steps(1, dt)
+            assert np.array_equal(s.get_state(), want)
+        s.set_state(JQ)
+        s.rk_step_record(dt, 0)
+        s.set_state(JQ)
+        s.rk_step_record(dt, 1)
+        s.steps(3, dt)
+        assert np.array_equal(s.get_state(), want)
