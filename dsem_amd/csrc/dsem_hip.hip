@@ -200,8 +200,20 @@ __device__ __forceinline__ size_t e2n_off(int n, int rot, int vq)
 
 // An element face's part in its mortar: it is the slave; its state is the left
 // one of the Roe flux; the slave's viscous trace changes sign; the mortar flux
-// changes sign on this face.
-enum { EF_SLAVE = 1, EF_LEFT = 2, EF_FLIP = 4, EF_NEG = 8 };
+// changes sign on this face; it does on the mortar's slave face.
+enum { EF_SLAVE = 1, EF_LEFT = 2, EF_FLIP = 4, EF_NEG = 8, EF_SIGN = 16 };
+
+// Adjoint of the viscous trace over the face norm, r / norm, at a face point:
+// -nu/2 times the adjoint of the mortar's flux, own + sign nbr on the master and
+// nbr + sign own on the slave, with the slave trace's sign (fl: EF_* bits; own,
+// nbr: adjoints of the two faces' fluxes).  The norms of k_update's flux and of
+// the trace cancel.
+__device__ __forceinline__ double visc_trace_adjoint(int fl, double inv_re, double own, double nbr)
+{
+    const bool slave = fl & EF_SLAVE, neg = fl & EF_SIGN;
+    const double s = (slave && neg ? -own : own) + (!slave && neg ? -nbr : nbr);
+    return (slave && (fl & EF_FLIP) ? 0.5 : -0.5) * inv_re * s;
+}
 
 // ------------------------------------------------------------ pointwise physics
 // Pointwise physics.  Euler fluxes: fflux/gflux/hflux (PhysLib.f90:17-124).
@@ -1637,8 +1649,8 @@ struct dsem_ctx {
     double *ev_rhos = nullptr;                 // density sensor at the Gauss points (k_ev)
     double *bmat = nullptr, *diag_part = nullptr, *diag_out = nullptr;   // diagnostics
     // adjoint buffers (allocated by the first VJP call)
-    double *aQVb = nullptr, *aGVb = nullptr, *aFTbe = nullptr, *aFVb = nullptr, *aQAbe = nullptr;
-    double *aTb = nullptr, *aFIb = nullptr, *aJQvb = nullptr, *aNuPart = nullptr, *aNu = nullptr;
+    double *aQVb = nullptr, *aGVb = nullptr, *aFTbe = nullptr, *aQAbe = nullptr;
+    double *aTb = nullptr, *aJQvb = nullptr, *aNuPart = nullptr, *aNu = nullptr;
     double *aGb = nullptr, *aLam = nullptr, *aOut = nullptr;
     double *aMuB = nullptr, *aWB = nullptr, *aSlagB = nullptr;   // entropy-viscosity adjoint (shock = 1)
     double *aNutB = nullptr;                   // Smagorinsky adjoint: that of the staggered nu_t
@@ -1986,10 +1998,8 @@ int adjoint_alloc(dsem_ctx *c)
         TRY(dev_alloc(c, &c->aQVb, K * 3 * NEQ * c->ns));
         TRY(dev_alloc(c, &c->aGVb, K * 3 * 15 * c->ns));
     }
-    TRY(dev_alloc(c, &c->aFVb, nfe));
     TRY(dev_alloc(c, &c->aQAbe, nfe));
     TRY(dev_alloc(c, &c->aTb, nfe));
-    TRY(dev_alloc(c, &c->aFIb, (size_t)c->M * NEQ * c->nf));
     TRY(dev_alloc(c, &c->aJQvb, n));
     TRY(dev_alloc(c, &c->aNuPart, K + face_blocks));
     TRY(dev_alloc(c, &c->aNu, 16));
@@ -2066,11 +2076,10 @@ int run_rhs_vjp(dsem_ctx *c, double *JQ, FwdTape f, bool fwd, double *Gb, double
     TRY(adj_volume_grid_size<P>(c, grid));
     return launch(c, KID_ADJ, [&] {
         k_adj_update<P><<<K, BLOCK, 0, s>>>(Gb, Qb, cdt, c->aFTbe);
-        k_adj_face_visc<P><<<face_blocks, BLOCK, 0, s>>>(c->aFTbe, f.FV, m, ph, c->aFIb, c->aFVb, nu_f);
         if constexpr (Vol<P>::MF) {
             auto vol = [&](auto model) {
                 k_adj_volume_mf<P, decltype(model)::value><<<grid, AdjVol<P>::BLK, 0, s>>>(
-                    JQ, m, ph, f.T, muh, Gb, c->aFVb, c->aJQvb, c->aQAbe, nu_v, MuB, SlagB, nut, NutB);
+                    JQ, m, ph, f.T, muh, Gb, c->aFTbe, c->aJQvb, c->aQAbe, nu_v, MuB, SlagB, nut, NutB);
             };
             if (nut && muh) vol(std::integral_constant<int, 3>{});
             else if (nut) vol(std::integral_constant<int, 2>{});
@@ -2079,7 +2088,7 @@ int run_rhs_vjp(dsem_ctx *c, double *JQ, FwdTape f, bool fwd, double *Gb, double
         } else {
             auto vol = [&](auto rot, auto lag) {
                 k_adj_volume<P, (P >= 4), decltype(rot)::value, decltype(lag)::value><<<K, ABLOCK, 0, s>>>(
-                    JQ, m, ph, f.T, muh, Gb, c->aFVb, c->aQVb, c->aGVb, nu_v, MuB, SlagB, nut, NutB);
+                    JQ, m, ph, f.T, muh, Gb, c->aFTbe, c->aQVb, c->aGVb, nu_v, MuB, SlagB, nut, NutB);
             };
             auto lagged = [&](auto rot) {
                 if (nut) vol(rot, std::integral_constant<int, 2>{});
@@ -2090,7 +2099,7 @@ int run_rhs_vjp(dsem_ctx *c, double *JQ, FwdTape f, bool fwd, double *Gb, double
             else lagged(std::false_type{});
             k_adj_gather<P><<<K, GBLOCK, 0, s>>>(m, c->aQVb, c->aGVb, c->aJQvb, c->aQAbe);
         }
-        k_adj_face_inv<P><<<face_blocks, BLOCK, 0, s>>>(f.T, m, ph, c->aFIb, c->aQAbe, c->aTb);
+        k_adj_face<P><<<face_blocks, BLOCK, 0, s>>>(f.T, f.FV, m, ph, c->aFTbe, c->aQAbe, c->aTb, nu_f);
         k_adj_traces<P><<<K, BLOCK, 0, s>>>(c->aTb, c->aJQvb, m, Out, Qb, Gb, a, c->aNuPart, face_blocks + K, nu_slot);
     });
 }
@@ -2579,7 +2588,7 @@ int create_impl(const dsem_mesh_desc *mesh, const dsem_params *prm, int device, 
             const size_t own = (size_t)el[s] * 6 + fa[s] - 1, nbr = (size_t)el[1 - s] * 6 + fa[1 - s] - 1;
             e2n[own] = (int)(nbr << 3) | (s == 0 ? mor[k] : ((e2m[own] >> 1) & 7));
             eflag[own] = (s ? EF_SLAVE : 0) | ((s == 0) != swap ? EF_LEFT : 0) | (mns[k] == -1 ? EF_FLIP : 0) |
-                         (s && msg[k] == -1 ? EF_NEG : 0);
+                         (s && msg[k] == -1 ? EF_NEG : 0) | (msg[k] == -1 ? EF_SIGN : 0);
         }
     }
 

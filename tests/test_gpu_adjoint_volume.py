@@ -1,6 +1,7 @@
 """Reverse volume kernel over the instances it comes in at p >= 5: each order
 without and with the model viscosities, and on more elements than workgroups
-are resident (a workgroup loops over elements).
+are resident (a workgroup loops over elements); the reverse of the face fluxes
+at every order on faces of all orientations.
 
 Central differences bound the error as in the other adjoint tests, 1e-6
 relative: with steps of 1e-6 (1e-7 where a viscosity's switches lie near) the
@@ -10,6 +11,7 @@ import numpy as np
 import pytest
 
 from dsem_amd import cases
+from dsem_amd import mesh as M
 from dsem_amd.solver import DSEM
 from helpers import distorted_box, graded_box, periodic_state
 
@@ -78,3 +80,29 @@ def test_gradient_of_every_viscosity_instance(p, ev, les):
         h = 1e-7 if ev else 1e-6
         d = np.random.default_rng(p).standard_normal(JQ.shape) * np.abs(JQ).mean(axis=(0, 2), keepdims=True)
         assert _close(float(np.sum(g * d)), (Jf(JQ + h * d) - Jf(JQ - h * d)) / (2 * h))
+
+
+@pytest.mark.parametrize("p", range(1, 9))
+def test_face_flux_adjoint_on_rotated_faces(p):
+    print(f"\n[case] reverse face fluxes p={p}", flush=True)
+    mesh = M.rotated_box(3, p, seed=p)
+    rng = np.random.default_rng(p)
+    nu, h = 1.0 / 200.0, 1e-6
+    with DSEM(mesh, re=1.0 / nu) as s:
+        xg, jac = s.gauss_points()
+        JQ = cases.tgv_state(xg, jac, "isothermal", perturb=2e-2, seed=p)
+        lam = rng.standard_normal(JQ.shape)
+        v = rng.standard_normal(JQ.shape) * np.abs(JQ).mean(axis=(0, 2), keepdims=True)
+        s.set_state(JQ)
+        jb, nub = s.rhs_vjp(lam)
+        s.set_state(JQ + h * v)
+        rp = s.rhs()
+        s.set_state(JQ - h * v)
+        rm = s.rhs()
+        assert _close(float(np.sum(jb * v)), float(np.sum(lam * (rp - rm)) / (2 * h)))
+    r = []
+    for f in (1.5, 0.5):   # R is linear in nu: any step will do
+        with DSEM(mesh, re=1.0 / (f * nu)) as s:
+            s.set_state(JQ)
+            r.append(s.rhs())
+    assert _close(nub, float(np.sum(lam * (r[0] - r[1])) / nu))
