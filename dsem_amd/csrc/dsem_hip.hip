@@ -1639,8 +1639,8 @@ struct dsem_ctx {
     double *Slag = nullptr, *muhg = nullptr, *ev_resid = nullptr, *ev_ducros = nullptr;   // entropy viscosity
     bool have_lag = false;
     bool keep_lag = false;                     // save the last stage's staggered states without EV
-    bool traces_cur = false;                   // T holds the face traces of the current JQ
-    bool state_lent = false;                   // dsem_state_pointers gave JQ out: a caller may write it
+    bool traces_cur = false;                   // T holds the face traces of JQ as the library last wrote it
+    bool state_lent = false;                   // dsem_state_pointers gave JQ out: see traces_valid
     int vol_grid = 0, adj_vol_grid = 0;        // resident workgroups of the persistent FP64 volume kernels
     bool les = false;                          // static Smagorinsky model
     double les_cs = 0.0, les_numax = 0.0;
@@ -2168,6 +2168,11 @@ int les_vjp_dispatch(dsem_ctx *c, const double *JQ, const double *Slag, double c
     DISPATCH_P(c, run_les_vjp, JQ, Slag, cs, numax, sensors, NutB, JQb, SlagB, nu_slot);
 }
 
+// T holds the face traces of JQ as it is now.  Once dsem_state_pointers has
+// given JQ out, its caller may write it between any two calls, so no call
+// starts from the traces that an earlier one left.
+bool traces_valid(const dsem_ctx *c) { return c->traces_cur && !c->state_lent; }
+
 // Tape layout per slot and stage: state [n], T [nT], FV [nT].
 size_t tape_stage_size(const dsem_ctx *c)
 {
@@ -2239,7 +2244,7 @@ int record_step(dsem_ctx *c, double dt, int slot)
 {
     const size_t n = (size_t)c->K * NEQ * c->np;
     int rc = DSEM_OK;
-    const bool ready = c->traces_cur && !c->state_lent;   // c->T holds the traces of c->JQ
+    const bool ready = traces_valid(c);
     if (c->les != c->tape_les)
         return set_err(c, DSEM_ERR_ARG, "the Smagorinsky switch changed since dsem_tape_reserve: reserve again");
     const bool lag_model = c->params.shock || c->les;
@@ -2297,7 +2302,7 @@ int record_step(dsem_ctx *c, double dt, int slot)
         rc = rhs_dispatch(c, S, st, nullptr, k > 0 || ready, true, (lag_model || c->keep_lag) && k == 4, &b);
     }
     if (rc == DSEM_OK && (lag_model || c->keep_lag)) c->have_lag = true;
-    c->traces_cur = rc == DSEM_OK && !c->state_lent;
+    c->traces_cur = rc == DSEM_OK;
     return rc;
 }
 
@@ -3056,10 +3061,10 @@ int dsem_rk_steps(dsem_ctx *c, double t, double dt, int nsteps, double *resid_ou
             st.resid = last ? &c->d_scalars[0] : nullptr;
             st.nonfinite = check ? reinterpret_cast<unsigned int *>(&c->d_scalars[2]) : nullptr;
             // The first stage needs the traces of the state: left in T by the
-            // previous call's last stage unless the state or T changed since.
+            // previous call's last stage unless the state or T may have changed since.
             // Every stage's update, the last included, leaves the traces of the
             // updated state for the next stage or call.
-            const bool ready = (s == 0 && k == 0) ? c->traces_cur : true;
+            const bool ready = (s == 0 && k == 0) ? traces_valid(c) : true;
             TRY(rhs_dispatch(c, c->JQ, st, nullptr, ready, true, (c->params.shock || c->keep_lag || c->les) && k == 4));
             std::swap(c->T, c->Tnext);
         }

@@ -316,6 +316,10 @@ int  dsem_rhs_device(dsem_ctx *ctx, const double *dJQ, double *dQt);
 #define DSEM_NOALLOC_SCRATCH_BYTES (64ull << 20)
 int  dsem_rhs_device_noalloc(dsem_ctx *ctx, const double *dJQ, double *dQt);
 
+/* The context's own state and RK register [K][5][ncg^3] (either nullable).
+ * The state may be written through dJQ, in the order of the context's stream:
+ * from this call on every step call recomputes the face traces of the state
+ * it starts from (one more kernel per call, not per step). */
 int  dsem_state_pointers(dsem_ctx *ctx, double **dJQ, double **dG);
 int  dsem_stream(dsem_ctx *ctx, void **hip_stream);
 int  dsem_synchronize(dsem_ctx *ctx);
