@@ -16,6 +16,7 @@ import numpy as np
 HERE = os.path.dirname(os.path.abspath(__file__))
 LIB_PATH = os.path.join(HERE, "liboracle.so")
 REF_PATH = os.path.join(HERE, "_ref", "libdsemref.so")
+REFERENCE = "/root/reference"
 
 _dp = C.POINTER(C.c_double)
 _ip = C.POINTER(C.c_int32)
@@ -46,7 +47,8 @@ def build(quiet: bool = True) -> None:
     out = subprocess.run(["make", "-C", HERE, "liboracle.so"], capture_output=True, text=True)
     if out.returncode:
         raise RuntimeError("oracle build failed:\n" + out.stdout + out.stderr)
-    if os.path.isdir("/root/reference"):
+    # an empty directory holds no sources
+    if os.path.exists(os.path.join(REFERENCE, "caseFiles", "tgv", "size.f90")):
         out = subprocess.run(["make", "-C", HERE, "ref"], capture_output=True, text=True)
         if out.returncode:
             raise RuntimeError("reference harness build failed:\n" + out.stdout + out.stderr)
