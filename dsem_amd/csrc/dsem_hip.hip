@@ -158,7 +158,7 @@ __device__ __forceinline__ int gidx(int d, int k, int a, int b)
 
 // face (1..6) reached at Lobatto end j of grid d
 template <int P>
-__device__ __forceinline__ int face_of(int d, int j)
+__host__ __device__ constexpr __forceinline__ int face_of(int d, int j)
 {
     const bool hi = (j != 0);
     return d == 0 ? (hi ? 4 : 6) : (d == 1 ? (hi ? 2 : 1) : (hi ? 5 : 3));
@@ -446,6 +446,16 @@ __device__ __forceinline__ double mf_line(const double *fld, const MfLane<P, ROW
     return t;
 }
 
+// Face whose averages the lane of row j of a grid-D line loads: the row's own
+// face, at interior rows one of another grid.  In grid D's pass the traces of
+// its two faces take the averages' place, so a lane that only keeps the
+// loads uniform must not touch those.
+template <int P, int D>
+__host__ __device__ constexpr __forceinline__ int average_face(int j)
+{
+    return j == 0 ? face_of<P>(D, 0) : (j == Sz<P>::NC - 1 ? face_of<P>(D, j) : face_of<P>((D + 2) % 3, 0));
+}
+
 // One staggered grid D of the mixed-precision volume kernel: fluxes at the
 // nc*ncg^2 points of grid D into LDS (interior) or the viscous face traces
 // (faces).
@@ -499,21 +509,21 @@ __device__ __forceinline__ void volume_grid(const DevMesh &m, const DevPhys &ph,
             else { a = s0 % S::NCG; b = (s0 / S::NCG) % S::NCG; j = s0 / (S::NCG * S::NCG); }
         }
         const int q = a + S::NCG * b;
-        const int jc = valid ? j : 0;
+        const int jc = valid ? j : 1;   // lanes without a point: an interior one
         const int s = sidx<P>(D, jc, a, b);
         const bool face = (jc == 0 || jc == S::NC - 1);
         const int fc = face_of<P>(D, jc);
         const int mo = e2m_mortar(e2m_e[fc - 1]);
         const int qm = m.rot ? orient_point<S::NCG>(e2m_map(e2m_e[fc - 1]), q) : q;   // the face point on the mortar
-        // The point's metric row, and its line's face average and norm (every
-        // lane: face_of names a face for any j, and interior lanes hit the
-        // face lane's cache lines), requested before the contractions instead
-        // of one wait each at their use
+        // The point's metric row, face average and norm, requested before the
+        // contractions instead of one wait each at their use; every lane
+        // loads, and interior ones keep nothing
         double vg[3] = {0.0, 0.0, 0.0}, vqa[5] = {0.0, 0.0, 0.0, 0.0, 0.0}, vnrm = 1.0;
+        const double *qa = FV + (size_t)e * 6 * NEQ * S::NF + ((average_face<P, D>(jc) - 1) * NEQ * S::NF + q);
 #pragma unroll
         for (int i = 0; i < 3; ++i) vg[i] = gmd[i * nsm + s * m.ms];
 #pragma unroll
-        for (int v = 0; v < 5; ++v) vqa[v] = FV[(((size_t)e * 6 + fc - 1) * NEQ + v) * S::NF + q];
+        for (int v = 0; v < 5; ++v) vqa[v] = qa[v * S::NF];
         vnrm = m.norm[(size_t)mo * nfm + qm * m.ms];
         double Qv[5];
         CT Bj[S::NCG];
