@@ -456,6 +456,15 @@ __host__ __device__ constexpr __forceinline__ int average_face(int j)
     return j == 0 ? face_of<P>(D, 0) : (j == Sz<P>::NC - 1 ? face_of<P>(D, j) : face_of<P>((D + 2) % 3, 0));
 }
 
+// The mixed-precision kernel keeps the FP64 face averages in LDS where that is
+// the faster place: p = 1, 2 and 4 to 6.  Elsewhere they wait in FV, where the
+// face points' traces will go: at p = 8 the LDS of a second workgroup on the CU
+// would be gone (95 KB each).  FP32 steps with FV and with LDS, us: 20^3
+// elements p = 1 731 and 674, p = 4 1698 and 1614; 18^3 p = 5 1612 and 1521; 16^3
+// p = 3 546 and 558, p = 6 1457 and 1342; 1320 elements p = 7 686 and 694.
+template <int P>
+constexpr bool averages_in_lds() { return P <= 6 && P != 3; }
+
 // One staggered grid D of the mixed-precision volume kernel: fluxes at the
 // nc*ncg^2 points of grid D into LDS (interior) or the viscous face traces
 // (faces).
@@ -465,8 +474,8 @@ __device__ __forceinline__ void volume_grid(const DevMesh &m, const DevPhys &ph,
                                             double *FV, double *__restrict__ Slag,
                                             const typename Ctr<PM>::T *sQ,
                                             const typename Ctr<PM>::T *sG, typename Ctr<PM>::T *sF,
-                                            const double *sBar, const typename Ctr<PM>::T *sB, int e,
-                                            const int *e2m_e, int tid)
+                                            const double *sBar, const double *sAv,
+                                            const typename Ctr<PM>::T *sB, int e, const int *e2m_e, int tid)
 {
     using S = Sz<P>;
     using CT = typename Ctr<PM>::T;
@@ -516,14 +525,16 @@ __device__ __forceinline__ void volume_grid(const DevMesh &m, const DevPhys &ph,
         const int mo = e2m_mortar(e2m_e[fc - 1]);
         const int qm = m.rot ? orient_point<S::NCG>(e2m_map(e2m_e[fc - 1]), q) : q;   // the face point on the mortar
         // The point's metric row, face average and norm, requested before the
-        // contractions instead of one wait each at their use; every lane
+        // contractions instead of one wait each at their use (from LDS too: p = 6
+        // 1342 us a step, 1356 with the average read at its use); every lane
         // loads, and interior ones keep nothing
         double vg[3] = {0.0, 0.0, 0.0}, vqa[5] = {0.0, 0.0, 0.0, 0.0, 0.0}, vnrm = 1.0;
+        constexpr bool AVL = averages_in_lds<P>();
         const double *qa = FV + (size_t)e * 6 * NEQ * S::NF + ((average_face<P, D>(jc) - 1) * NEQ * S::NF + q);
 #pragma unroll
         for (int i = 0; i < 3; ++i) vg[i] = gmd[i * nsm + s * m.ms];
 #pragma unroll
-        for (int v = 0; v < 5; ++v) vqa[v] = qa[v * S::NF];
+        for (int v = 0; v < 5; ++v) vqa[v] = AVL ? sAv[((fc - 1) * NEQ + v) * S::NF + q] : qa[v * S::NF];
         vnrm = m.norm[(size_t)mo * nfm + qm * m.ms];
         double Qv[5];
         CT Bj[S::NCG];
@@ -711,6 +722,7 @@ __global__ __launch_bounds__(VBLOCK, 4) void k_volume(const double *__restrict__
     // gradient phase it holds the face averages of the six faces
     constexpr int NSF = NEQ * S::NS > 6 * NEQ * S::NF ? NEQ * S::NS : 6 * NEQ * S::NF;
     __shared__ CT sF[NSF];
+    __shared__ double sAv[averages_in_lds<P>() ? 6 * NEQ * S::NF : 1];   // face averages, FP64
     __shared__ double sBar[5 + 15];           // Qbar[5], Fbar[3][5]
     // operator matrices of this order: M = D_int B (Gauss derivative), D, B
     constexpr int OM = 0, OD = S::NCG * S::NCG, OB = OD + S::NCG * S::NC, NOP = OB + S::NC * S::NCG;
@@ -796,8 +808,8 @@ __global__ __launch_bounds__(VBLOCK, 4) void k_volume(const double *__restrict__
         if (i < NAV) {
             const double a = in.face(u);
             sQA[i] = (CT)(a - sBar[(i % NFV) / S::NF]);
-            // the FP64 averages wait where the face points' traces will go
-            FV[(size_t)e * NAV + i] = a;
+            if constexpr (averages_in_lds<P>()) sAv[i] = a;
+            else FV[(size_t)e * NAV + i] = a;
         }
     }
     __syncthreads();
@@ -845,11 +857,11 @@ __global__ __launch_bounds__(VBLOCK, 4) void k_volume(const double *__restrict__
     for (int r = 0; r < R; ++r)
 #pragma unroll
         for (int v = 0; v < 5; ++v) acc[r][v] = 0.0;
-    volume_grid<P, 0, PM>(m, ph, muh, nut, FV, Slag, sQ, sG, sF, sBar, sOp + OB, e, e2m_e, tid);
+    volume_grid<P, 0, PM>(m, ph, muh, nut, FV, Slag, sQ, sG, sF, sBar, sAv, sOp + OB, e, e2m_e, tid);
     volume_div<P, 0, PM>(sF, sOp + OD, sBar, sDint, tid, acc);
-    volume_grid<P, 1, PM>(m, ph, muh, nut, FV, Slag, sQ, sG, sF, sBar, sOp + OB, e, e2m_e, tid);
+    volume_grid<P, 1, PM>(m, ph, muh, nut, FV, Slag, sQ, sG, sF, sBar, sAv, sOp + OB, e, e2m_e, tid);
     volume_div<P, 1, PM>(sF, sOp + OD, sBar, sDint, tid, acc);
-    volume_grid<P, 2, PM>(m, ph, muh, nut, FV, Slag, sQ, sG, sF, sBar, sOp + OB, e, e2m_e, tid);
+    volume_grid<P, 2, PM>(m, ph, muh, nut, FV, Slag, sQ, sG, sF, sBar, sAv, sOp + OB, e, e2m_e, tid);
     volume_div<P, 2, PM>(sF, sOp + OD, sBar, sDint, tid, acc);
 #pragma unroll
     for (int r = 0; r < R; ++r) {
