@@ -2109,7 +2109,7 @@ int run_rhs_vjp(dsem_ctx *c, double *JQ, FwdTape f, bool fwd, double *Gb, double
             else vol(std::integral_constant<int, 0>{});
         } else {
             auto vol = [&](auto rot, auto lag) {
-                k_adj_volume<P, (P >= 4), decltype(rot)::value, decltype(lag)::value><<<K, ABLOCK, 0, s>>>(
+                k_adj_volume<P, (P >= 4), decltype(rot)::value, decltype(lag)::value><<<K, ablock<P>(), 0, s>>>(
                     JQ, m, ph, f.T, muh, Gb, c->aFTbe, c->aQVb, c->aGVb, nu_v, MuB, SlagB, nut, NutB);
             };
             auto lagged = [&](auto rot) {
