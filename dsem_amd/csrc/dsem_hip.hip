@@ -705,7 +705,7 @@ __device__ __forceinline__ void volume_div(const typename Ctr<PM>::T *sF, const 
 //   flux  F - Fbar_d (Fbar_d = contravariant Euler flux of Qbar with the
 //         metric row at staggered point 0 of grid d); the divergence adds
 //         Fbar_d * sum_{interior j} D[k][j] back in FP64.
-// Pointwise physics, the RK state and all face kernels stay FP64.
+// Pointwise physics, the RK state and the face fluxes stay FP64.
 template <int P, int PM>
 __global__ __launch_bounds__(VBLOCK, 4) void k_volume(const double *__restrict__ JQ, DevMesh m, DevPhys ph,
                                                       const double *__restrict__ T, const double *__restrict__ muh,
@@ -1809,10 +1809,11 @@ int volume_grid_size(dsem_ctx *c, int &grid)
     return DSEM_OK;
 }
 
-// Per-call intermediates of one RHS evaluation: face traces T, mortar
-// averages QA, Roe fluxes FI, viscous face traces FV, total face fluxes FT
-// and the partial residual Qtp.  Every entry a call reads is written earlier
-// in the same call, so none needs clearing.
+// Arrays of one RHS evaluation: face traces T of its state, viscous face traces
+// FV and the partial residual Qtp; an RK stage leaves the traces of the updated
+// state in Tnext (neighbours still read T).  Every entry a call reads is
+// written earlier in the same call (T perhaps by the call before), so none
+// needs clearing.
 struct RhsBufs {
     double *T, *Tnext, *FV, *Qtp;
     double *JQnext = nullptr;   // where an RK stage leaves the state, null: in place
